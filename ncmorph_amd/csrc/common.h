@@ -71,6 +71,26 @@ __device__ __forceinline__ void swiglu_bits2(float ga0, float ua0, float ga1, fl
     o1 = r >> 16;
 }
 
+// rotate_head in bf16 mode (packages/kernels/root.zig:615-634) of two
+// elements at once: a and b hold the bf16 bits of a head's first- and
+// second-half elements (one per 16-bit half), tc / ts and tc2 / ts2 the
+// rounded cosines and sines of their two table columns. left = rb(a rb(cos)),
+// right = rb(-b rb(sin)), right2 = rb(a rb(sin2)), left2 = rb(b rb(cos2)),
+// then a = round(left + right), b = round(left2 + right2). Intermediates go
+// without the NaN rule (a NaN stays a NaN through products and sums; the
+// final rounding maps it to 0x7FC0).
+__device__ __forceinline__ void rope_bits2(uint32_t& a, uint32_t& b, uint32_t tc, uint32_t ts,
+                                           uint32_t tc2, uint32_t ts2) {
+    auto lo = [](uint32_t p) { return __uint_as_float(p << 16); };
+    auto hi = [](uint32_t p) { return __uint_as_float(p & 0xFFFF0000u); };
+    const uint32_t left = bf16x2_rne(lo(a) * lo(tc), hi(a) * hi(tc));
+    const uint32_t right = bf16x2_rne(-lo(b) * lo(ts), -hi(b) * hi(ts));
+    const uint32_t right2 = bf16x2_rne(lo(a) * lo(ts2), hi(a) * hi(ts2));
+    const uint32_t left2 = bf16x2_rne(lo(b) * lo(tc2), hi(b) * hi(tc2));
+    a = bf16x2_bits_rne(lo(left) + lo(right), hi(left) + hi(right));
+    b = bf16x2_bits_rne(lo(left2) + lo(right2), hi(left2) + hi(right2));
+}
+
 __device__ __forceinline__ float bf16_lo_to_f32(uint32_t packed) {
     return __uint_as_float(packed << 16);
 }

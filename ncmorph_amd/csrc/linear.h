@@ -53,6 +53,22 @@ hipError_t launch_linear_tail(const uint16_t* x, const uint16_t* w, const uint16
                               const float* residual, void* y, int64_t R, int64_t K, int64_t N,
                               int out_mode, bool swiglu, hipStream_t st);
 
+// Few rows (linear_slice.hip): whether the K-sliced kernel takes an M x N x K
+// bf16 product (launch_linear, launch_linear_residual, launch_linear_swiglu
+// and launch_linear_rope64 all ask this, with N the weight's rows), and its
+// launchers, with those functions' arguments.
+bool linear_slice_fits(int64_t M, int64_t N, int64_t K);
+hipError_t launch_linear_slice(const uint16_t* x, const uint16_t* w, const uint16_t* bias,
+                               const float* residual, void* y, int64_t M, int64_t K, int64_t N,
+                               int out_mode, hipStream_t stream);
+hipError_t launch_linear_slice_swiglu(const uint16_t* x, const uint16_t* w, const uint16_t* bias,
+                                      uint16_t* y, int64_t M, int64_t K, int64_t N2,
+                                      hipStream_t stream);
+hipError_t launch_linear_slice_rope64(const uint16_t* x, const uint16_t* w, const uint16_t* bias,
+                                      uint16_t* y, int64_t M, int64_t K, int64_t N,
+                                      int64_t rot_cols, int64_t seq_len, const float* cosine,
+                                      const float* sine, hipStream_t stream);
+
 // fp32 operands, fp32 output; K % 4 == 0, 16-byte aligned x and w.
 hipError_t launch_linear_f32(const float* x, const float* w, float* y, int64_t M, int64_t K,
                              int64_t N, hipStream_t stream);

@@ -261,6 +261,8 @@ hipError_t launch_linear(const uint16_t* x, const uint16_t* w, const uint16_t* b
     }();
     if (config < 0) config = env_cfg;
     if (config < 0) {
+        if (linear_slice_fits(M, N, K))
+            return launch_linear_slice(x, w, bias, nullptr, y, M, K, N, out_mode, stream);
         // A partial last row tile that would add a round: its rows go to the
         // tail kernel.
         const int64_t r = linear_tail_rows(M, N, K);
@@ -311,8 +313,10 @@ static hipError_t launch_linear_res_s(const uint16_t* x, const uint16_t* w, cons
 hipError_t launch_linear_residual(const uint16_t* x, const uint16_t* w, const uint16_t* bias,
                                   const float* residual, void* y, int64_t M, int64_t K,
                                   int64_t N, int out_mode, hipStream_t stream) {
-    // The automatic tile choice only (configurations 0, 1, 2 and 5), with
-    // the tail rows of linear_tail_rows on the tail kernel.
+    // The automatic choice only: the K-sliced kernel, or configurations 0, 1,
+    // 2 and 5 with the tail rows of linear_tail_rows on the tail kernel.
+    if (linear_slice_fits(M, N, K))
+        return launch_linear_slice(x, w, bias, residual, y, M, K, N, out_mode, stream);
     const int64_t r = linear_tail_rows(M, N, K);
     if (r > 0) {
         const int64_t mm = M - r;

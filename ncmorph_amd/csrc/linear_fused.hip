@@ -130,11 +130,12 @@ __attribute__((amdgpu_waves_per_eu(S::OCC, S::OCC))) void linear_pair_kernel(
                 }
                 quad_transpose4(va, q);
                 quad_transpose4(vb, q);
-                uint32_t ra[4], rbits[4];
+                // Two columns per register from here on.
+                uint32_t ra[2], rbits[2];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    ra[j] = __float_as_uint(va[j]);
-                    rbits[j] = __float_as_uint(vb[j]);
+                for (int h = 0; h < 2; ++h) {
+                    ra[h] = __float_as_uint(va[2 * h]) | (__float_as_uint(va[2 * h + 1]) << 16);
+                    rbits[h] = __float_as_uint(vb[2 * h]) | (__float_as_uint(vb[2 * h + 1]) << 16);
                 }
                 if (rotate) {
                     const int64_t t = (m < M ? m : 0) % pa.seq_len;
@@ -142,48 +143,21 @@ __attribute__((amdgpu_waves_per_eu(S::OCC, S::OCC))) void linear_pair_kernel(
                     const f32x4_t cs = *(const f32x4_t*)(pa.cosine + t * 64 + 32 + c4);
                     const f32x4_t sf = *(const f32x4_t*)(pa.sine + t * 64 + c4);
                     const f32x4_t ss = *(const f32x4_t*)(pa.sine + t * 64 + 32 + c4);
-                    // Per column: left = rb(first rb(cos)), right =
-                    // rb(-second rb(sin)), right2 = rb(first rb(sin2)),
-                    // left2 = rb(second rb(cos2)), then round(left + right)
-                    // and round(left2 + right2); each rounding done for two
-                    // columns at once (bf16x2_bits_rne, the bits of rb).
-                    auto lo = [](uint32_t pr) { return __uint_as_float(pr << 16); };
-                    auto hi = [](uint32_t pr) { return __uint_as_float(pr & 0xFFFF0000u); };
 #pragma unroll
-                    for (int j = 0; j < 4; j += 2) {
-                        const float f0 = __uint_as_float(ra[j] << 16);
-                        const float f1 = __uint_as_float(ra[j + 1] << 16);
-                        const float s0 = __uint_as_float(rbits[j] << 16);
-                        const float s1 = __uint_as_float(rbits[j + 1] << 16);
-                        // Intermediates without the NaN rule (a NaN stays a
-                        // NaN through products and sums; the final rounding
-                        // maps it to 0x7FC0).
-                        const uint32_t tc = bf16x2_rne(cf[j], cf[j + 1]);
-                        const uint32_t ts = bf16x2_rne(sf[j], sf[j + 1]);
-                        const uint32_t ts2 = bf16x2_rne(ss[j], ss[j + 1]);
-                        const uint32_t tc2 = bf16x2_rne(cs[j], cs[j + 1]);
-                        const uint32_t left = bf16x2_rne(f0 * lo(tc), f1 * hi(tc));
-                        const uint32_t right = bf16x2_rne(-s0 * lo(ts), -s1 * hi(ts));
-                        const uint32_t right2 = bf16x2_rne(f0 * lo(ts2), f1 * hi(ts2));
-                        const uint32_t left2 = bf16x2_rne(s0 * lo(tc2), s1 * hi(tc2));
-                        const uint32_t o1 = bf16x2_bits_rne(lo(left) + lo(right),
-                                                            hi(left) + hi(right));
-                        const uint32_t o2 = bf16x2_bits_rne(lo(left2) + lo(right2),
-                                                            hi(left2) + hi(right2));
-                        ra[j] = o1 & 0xFFFFu;
-                        ra[j + 1] = o1 >> 16;
-                        rbits[j] = o2 & 0xFFFFu;
-                        rbits[j + 1] = o2 >> 16;
-                    }
+                    for (int h = 0; h < 2; ++h)
+                        rope_bits2(ra[h], rbits[h], bf16x2_rne(cf[2 * h], cf[2 * h + 1]),
+                                   bf16x2_rne(sf[2 * h], sf[2 * h + 1]),
+                                   bf16x2_rne(cs[2 * h], cs[2 * h + 1]),
+                                   bf16x2_rne(ss[2 * h], ss[2 * h + 1]));
                 }
                 if (m < M) {
                     u32x2_t o;
-                    o[0] = ra[0] | (ra[1] << 16);
-                    o[1] = ra[2] | (ra[3] << 16);
+                    o[0] = ra[0];
+                    o[1] = ra[1];
                     __builtin_nontemporal_store(o, (u32x2_t*)(y + m * ld + ca));
                     if (EPI == kEpiRope) {
-                        o[0] = rbits[0] | (rbits[1] << 16);
-                        o[1] = rbits[2] | (rbits[3] << 16);
+                        o[0] = rbits[0];
+                        o[1] = rbits[1];
                         __builtin_nontemporal_store(o, (u32x2_t*)(y + m * ld + ca + 32));
                     }
                 }
@@ -242,6 +216,8 @@ hipError_t launch_linear_swiglu(const uint16_t* x, const uint16_t* w, const uint
                                 uint16_t* y, int64_t M, int64_t K, int64_t N2,
                                 hipStream_t stream) {
     if (N2 % 64) return hipErrorInvalidValue;
+    if (linear_slice_fits(M, N2, K))
+        return launch_linear_slice_swiglu(x, w, bias, y, M, K, N2, stream);
     const int64_t r = linear_tail_rows(M, N2, K);
     if (r > 0) {
         const int64_t mm = M - r;
@@ -260,6 +236,9 @@ hipError_t launch_linear_rope64(const uint16_t* x, const uint16_t* w, const uint
                                 int64_t seq_len, const float* cosine, const float* sine,
                                 hipStream_t stream) {
     if (N % 64 || rot_cols % 64 || seq_len <= 0) return hipErrorInvalidValue;
+    if (linear_slice_fits(M, N, K))
+        return launch_linear_slice_rope64(x, w, bias, y, M, K, N, rot_cols, seq_len, cosine, sine,
+                                          stream);
     return launch_pair<kEpiRope>(x, w, bias, y, M, K, N,
                                  PairArgs{cosine, sine, seq_len, rot_cols}, stream);
 }

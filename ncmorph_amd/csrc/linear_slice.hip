@@ -1,0 +1,407 @@
+// Linears with few rows: y = x * W^T where the 128- and 256-row tiles of
+// linear.hip leave most of the chip idle or multiply mostly padding (a
+// prompt of 77 tokens through a 2048-wide projection is 16 tiles for 256
+// CUs). Small output tiles fill the CUs, and the wavefronts of a workgroup
+// split K instead of the tile: wavefront w multiplies the whole tile over
+// K tiles w, w + NW, ... (64 bf16 or 32 fp32 elements each) and the NW
+// partial sums are added in wavefront order through LDS at the end, so there
+// is no second pass over memory, no workspace and no atomic.
+//
+// What bounds it: the weight stream from HBM for the smallest batches, the
+// operand traffic L2 -> LDS (every column tile reads all of x, every row tile
+// all of W) for the larger ones. A wavefront's operand rows go straight to
+// its own LDS region (buffer_load ... lds, 8 rows x 128 bytes per
+// instruction: whole cache lines), NST stages deep. No other wavefront reads
+// that region, so the main loop has no barrier: each wavefront waits for its
+// oldest stage only (vmcnt), reads the stage's fragments into registers and
+// refills the stage before its MFMAs.
+//
+// Fragments: v_mfma_f32_16x16x32_bf16 (A = x rows, B = weight rows; lane l
+// supplies 16-byte chunk 4 i + l / 16 of row l % 16 for k-step i), or for
+// fp32 four v_mfma_f32_16x16x4_f32 per k-step, MFMA j taking element j of
+// each lane's chunk. D: lane l, element j holds row 4 (l / 16) + j, column
+// l % 16. LDS chunk c of row r sits at chunk c ^ ((r / 2) % 8), which gives
+// the 16 rows of a ds_read_b128 phase distinct bank groups.
+//
+// Every output is a function of its row of x and its weight row(s) alone,
+// and of K and NW, which launch_slice takes from (M, N, K): the same sums for
+// every epilogue, so the fused results equal the unfused kernels' bit for bit.
+#include "common.h"
+#include "gemm_core.h"
+#include "linear.h"
+
+namespace ncm {
+
+namespace {
+
+constexpr int kPlain = 0, kSwiGLU = 1, kRope = 2;
+
+struct SliceArgs {
+    const void* x;
+    const void* w;
+    const uint16_t* bias;  // bf16, nullable
+    const float* residual;  // fp32 [M, N], nullable; may be y in the fp32 modes
+    void* y;
+    int64_t M, K, N;  // N: weight rows
+    int out_mode, tiles_m;
+    // RoPE: tables [seq_len, 64], columns [0, rot_cols) rotated.
+    const float* cosine;
+    const float* sine;
+    int64_t seq_len, rot_cols;
+};
+
+// RB x CB blocks of 16 x 16 outputs per workgroup, NW wavefronts, NST LDS
+// stages each.
+template <bool F32, int RB, int CB, int NW, int NST>
+struct SliceShape {
+    static constexpr int ROWS = 16 * (RB + CB);
+    static constexpr int STAGE = ROWS * 128;
+    static constexpr int ND = ROWS / 8;  // load instructions per stage
+    static constexpr int RED = NW * RB * CB * 1024;
+    static constexpr int LDS = NW * NST * STAGE > RED ? NW * NST * STAGE : RED;
+    static constexpr int EPC = F32 ? 4 : 8;  // elements per 16-byte chunk
+    static_assert(LDS <= 160 * 1024, "LDS budget of a gfx950 CU");
+    static_assert(NST >= 1 && (NST - 1) * ND <= 63, "vmcnt range");
+};
+
+template <bool F32, int RB, int CB, int NW, int NST, int EPI>
+__global__ __launch_bounds__(64 * NW) void linear_slice_kernel(SliceArgs a) {
+    using S = SliceShape<F32, RB, CB, NW, NST>;
+    constexpr int ESZ = F32 ? 4 : 2;
+    constexpr int NB = RB * CB;
+    static_assert(EPI == kPlain || CB == 2 || CB == 4, "pairs of 16-column blocks");
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r16 = lane & 15, grp = lane >> 4;
+
+    // The row tiles of one column tile are consecutive and on one XCD (each
+    // XCD takes a contiguous run of tiles), so W is read from HBM once.
+    const int nblk = (int)gridDim.x, bid = (int)blockIdx.x;
+    const int xcd = bid & 7, per = nblk >> 3, rem = nblk & 7;
+    const int logical = xcd * per + min(xcd, rem) + (bid >> 3);
+    const int tm = logical % a.tiles_m;
+    const int tn = logical / a.tiles_m;
+
+    const int64_t m0 = (int64_t)tm * 16 * RB;
+    // First weight row. The paired epilogues (gate and up rows, or the two
+    // halves of a head) need rows c and c + 32 of a 64-row group together:
+    // CB = 4 takes the group, CB = 2 its rows s .. s + 15 and s + 32 .. s + 47.
+    const int64_t n0 = EPI == kPlain || CB == 4 ? (int64_t)tn * 16 * CB
+                                                : (int64_t)(tn >> 1) * 64 + (tn & 1) * 16;
+    constexpr int BSTEP = EPI != kPlain && CB == 2 ? 32 : 16;  // rows between column blocks
+    const int64_t K = a.K;
+    const __amdgpu_buffer_rsrc_t rsx =
+        make_rsrc((const char*)a.x + m0 * K * ESZ, operand_bytes(a.M, m0, K, ESZ));
+    const __amdgpu_buffer_rsrc_t rsw =
+        make_rsrc((const char*)a.w + n0 * K * ESZ, operand_bytes(a.N, n0, K, ESZ));
+
+    // Load instruction p fills LDS rows 8 p .. 8 p + 7 (x rows, then weight
+    // rows), lane l row l / 8, chunk slot l % 8; the swizzle term depends on
+    // the parity of p only.
+    const int drow = lane >> 3;
+    const int ch0 = (lane & 7) ^ (drow >> 1), ch1 = ch0 ^ 4;
+    const uint32_t rowb = (uint32_t)(K * ESZ);
+    const uint32_t o0 = drow * rowb + ch0 * 16, o1 = drow * rowb + ch1 * 16;
+    char* region = lds + wave * (NST * S::STAGE);
+    auto dma = [&](char* stage, int64_t k0) {
+        // Chunks at or past K, and tiles past the last one, load as zero.
+        const uint32_t kb = (uint32_t)(k0 * ESZ);
+        const uint32_t v0 = k0 + ch0 * S::EPC < K ? o0 + kb : kOobOffset;
+        const uint32_t v1 = k0 + ch1 * S::EPC < K ? o1 + kb : kOobOffset;
+#pragma unroll
+        for (int p = 0; p < S::ND; ++p) {
+            const bool is_x = p < 2 * RB;
+            const int q = is_x ? p : p - 2 * RB;
+            const int row = is_x ? 8 * q : (q >> 1) * BSTEP + 8 * (q & 1);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                is_x ? rsx : rsw,
+                (__attribute__((address_space(3))) void*)(stage + p * 1024), 16,
+                (p & 1 ? v1 : v0) + (uint32_t)row * rowb, 0, 0, 0);
+        }
+    };
+
+    f32x4_t acc[RB][CB];
+#pragma unroll
+    for (int i = 0; i < RB; ++i)
+#pragma unroll
+        for (int j = 0; j < CB; ++j) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+
+    constexpr int BK = 8 * S::EPC;
+    const int tiles_k = (int)((K + BK - 1) / BK);
+    const int iters = (tiles_k + NW - 1) / NW;
+#pragma unroll
+    for (int s = 0; s < NST; ++s) dma(region + s * S::STAGE, (int64_t)(wave + NW * s) * BK);
+    const uint32_t frag = (uint32_t)(r16 * 128);
+    const uint32_t c0 = (uint32_t)((grp ^ (r16 >> 1)) * 16), c1 = c0 ^ 64;
+    int st = 0;
+    for (int i = 0; i < iters; ++i) {
+        char* base = region + st * S::STAGE;
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0((NST - 1) * S::ND));
+        asm volatile("" ::: "memory");
+        u32x4_t af[2][RB], bf[2][CB];
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            const uint32_t c = ks ? c1 : c0;
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb)
+                af[ks][rb] = *(const u32x4_t*)(base + frag + rb * 2048 + c);
+#pragma unroll
+            for (int cb = 0; cb < CB; ++cb)
+                bf[ks][cb] = *(const u32x4_t*)(base + frag + (RB + cb) * 2048 + c);
+        }
+        // The stage is free once its fragments are in registers.
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        dma(base, (int64_t)(wave + NW * (i + NST)) * BK);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+                for (int cb = 0; cb < CB; ++cb) {
+                    if constexpr (F32) {
+#pragma unroll
+                        for (int j = 0; j < 4; ++j)
+                            acc[rb][cb] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                                __uint_as_float(af[ks][rb][j]), __uint_as_float(bf[ks][cb][j]),
+                                acc[rb][cb], 0, 0, 0);
+                    } else {
+                        acc[rb][cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            __builtin_bit_cast(bf16x8_t, af[ks][rb]),
+                            __builtin_bit_cast(bf16x8_t, bf[ks][cb]), acc[rb][cb], 0, 0, 0);
+                    }
+                }
+        st = st + 1 == NST ? 0 : st + 1;
+    }
+
+    // Partial sums over the operand stages, once no load can still write
+    // there; block b of wavefront v at ((v NB + b) 64 + lane) 16 bytes.
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    f32x4_t* red = (f32x4_t*)lds;
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb) red[(wave * NB + rb * CB + cb) * 64 + lane] = acc[rb][cb];
+    __syncthreads();
+    auto sum = [&](int b) {
+        f32x4_t s = red[b * 64 + lane];
+#pragma unroll
+        for (int v = 1; v < NW; ++v) {
+            const f32x4_t p = red[(v * NB + b) * 64 + lane];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) s[j] = s[j] + p[j];
+        }
+        return s;
+    };
+    auto bias_of = [&](int64_t n) {
+        return a.bias ? __uint_as_float((uint32_t)a.bias[n] << 16) : 0.0f;
+    };
+
+    if constexpr (EPI == kPlain) {
+        for (int b = wave; b < NB; b += NW) {
+            const int64_t n = n0 + 16 * (b % CB) + r16;
+            f32x4_t v = sum(b);
+            if (n >= a.N) continue;
+            const float bv = bias_of(n);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int64_t m = m0 + 16 * (b / CB) + 4 * grp + j;
+                if (m >= a.M) continue;
+                const int64_t off = m * a.N + n;
+                const float f = a.bias ? v[j] + bv : v[j];
+                if (a.out_mode == NCM_OUT_F32) {
+                    ((float*)a.y)[off] = a.residual ? a.residual[off] + f : f;
+                } else {
+                    uint32_t bits = bf16_bits_rne(flush_subnormal(f));
+                    if (a.residual)
+                        bits = bf16_bits_rne(a.residual[off] + __uint_as_float(bits << 16));
+                    if (a.out_mode == NCM_OUT_BF16_F32)
+                        ((float*)a.y)[off] = __uint_as_float(bits << 16);
+                    else
+                        ((uint16_t*)a.y)[off] = (uint16_t)bits;
+                }
+            }
+        }
+        return;
+    }
+    // Pairs: column blocks cb and cb + CB / 2, 32 weight rows apart.
+    constexpr int HB = CB > 1 ? CB / 2 : 1;
+    for (int b = wave; b < RB * HB; b += NW) {
+        const int rb = b / HB, cb = b % HB;
+        const f32x4_t va = sum(rb * CB + cb), vb = sum(rb * CB + cb + HB);
+        const int64_t na = n0 + 16 * cb + r16;  // N % 64 == 0: the pair is in range
+        const float ba = bias_of(na), bb = bias_of(na + 32);
+        uint16_t* y = (uint16_t*)a.y;
+#pragma unroll
+        for (int j = 0; j < 4; j += 2) {
+            const int64_t m = m0 + 16 * rb + 4 * grp + j;
+            if constexpr (EPI == kSwiGLU) {
+                uint32_t q0, q1;
+                swiglu_bits2(va[j], vb[j], va[j + 1], vb[j + 1], ba, bb, q0, q1);
+                const int64_t col = (na >> 6) * 32 + (na & 31);
+                if (m < a.M) y[m * (a.N / 2) + col] = (uint16_t)q0;
+                if (m + 1 < a.M) y[(m + 1) * (a.N / 2) + col] = (uint16_t)q1;
+            } else {
+                // Two rows of the projection's bits, bf16(flush(acc + bias)).
+                uint32_t fa = bf16x2_bits_rne(flush_subnormal(va[j] + ba),
+                                              flush_subnormal(va[j + 1] + ba));
+                uint32_t fb = bf16x2_bits_rne(flush_subnormal(vb[j] + bb),
+                                              flush_subnormal(vb[j + 1] + bb));
+                if (na < a.rot_cols) {
+                    const int c = (int)(na & 63);
+                    const float* ct0 = a.cosine + ((m < a.M ? m : 0) % a.seq_len) * 64 + c;
+                    const float* ct1 = a.cosine + ((m + 1 < a.M ? m + 1 : 0) % a.seq_len) * 64 + c;
+                    const float* st0 = a.sine + (ct0 - a.cosine);
+                    const float* st1 = a.sine + (ct1 - a.cosine);
+                    rope_bits2(fa, fb, bf16x2_rne(ct0[0], ct1[0]), bf16x2_rne(st0[0], st1[0]),
+                               bf16x2_rne(ct0[32], ct1[32]), bf16x2_rne(st0[32], st1[32]));
+                }
+                if (m < a.M) {
+                    y[m * a.N + na] = (uint16_t)fa;
+                    y[m * a.N + na + 32] = (uint16_t)fb;
+                }
+                if (m + 1 < a.M) {
+                    y[(m + 1) * a.N + na] = (uint16_t)(fa >> 16);
+                    y[(m + 1) * a.N + na + 32] = (uint16_t)(fb >> 16);
+                }
+            }
+        }
+    }
+}
+
+template <bool F32, int RB, int CB, int NW, int NST, int EPI>
+hipError_t launch_slice_t(SliceArgs a, hipStream_t st) {
+    using S = SliceShape<F32, RB, CB, NW, NST>;
+    auto kern = linear_slice_kernel<F32, RB, CB, NW, NST, EPI>;
+    static const hipError_t attr = hipFuncSetAttribute(
+        (const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, S::LDS);
+    if (attr != hipSuccess) return attr;
+    a.tiles_m = (int)((a.M + 16 * RB - 1) / (16 * RB));
+    const int64_t blocks = a.tiles_m * ((a.N + 16 * CB - 1) / (16 * CB));
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(64 * NW), S::LDS, st, a);
+    return hipGetLastError();
+}
+
+// Tiles RB x CB with their LDS stages. NW is 8 for all of them: the sums of
+// an output do not depend on the tile. One stage (refilled while its
+// fragments are multiplied) leaves LDS for a second workgroup on the CU up to
+// 5 blocks of rows and measured as fast as two or three from 1 x 2 up.
+constexpr int kSliceWaves = 8;
+struct Tile {
+    int rb, cb;
+};
+constexpr Tile kTiles[] = {{1, 1}, {2, 1}, {1, 2}, {2, 2}, {3, 2}, {1, 4},
+                           {4, 2}, {2, 4}, {3, 4}, {4, 4}, {5, 4}};
+constexpr int kTileCount = sizeof(kTiles) / sizeof(kTiles[0]);
+
+// Cost of a tile: rounds of the 256 CUs times the blocks of 16 operand rows
+// that a workgroup loads (at 75 GB/s a CU, over all shapes measured: 31 us for
+// 512 x 2048 x 8192 at cost 8, 18 us for 128 rows at cost 4).
+int64_t tile_cost(const Tile& s, int64_t M, int64_t N) {
+    const int64_t tiles =
+        ((M + 16 * s.rb - 1) / (16 * s.rb)) * ((N + 16 * s.cb - 1) / (16 * s.cb));
+    return (tiles + 255) / 256 * (s.rb + s.cb);
+}
+
+// The cheapest tile (paired: one with a partner column block).
+int64_t best_tile(int64_t M, int64_t N, bool paired, int* tile) {
+    int64_t best = INT64_MAX;
+    for (int t = 0; t < kTileCount; ++t) {
+        if (paired && kTiles[t].cb < 2) continue;
+        const int64_t cost = tile_cost(kTiles[t], M, N);
+        if (cost < best) {
+            best = cost;
+            *tile = t;
+        }
+    }
+    // Up to 48 rows against a head of four rounds or more: the weight stream
+    // is the bound, and two workgroups a CU with two column blocks each keep
+    // more of it in flight (24 rows, 151936 x 1024: 77 -> 70 us; 40 rows: 90 ->
+    // 77 us; 24 rows, 128256 x 2048: 116 -> 110 us).
+    const int64_t rb = (M + 15) / 16;
+    if (rb <= 3 && (N + 63) / 64 > 3 * 256) *tile = rb == 1 ? 2 : (rb == 2 ? 3 : 4);
+    return best;
+}
+
+template <int EPI>
+hipError_t launch_slice(int tile, const SliceArgs& a, hipStream_t st) {
+#define NCM_SLICE(RB, CB, NST) \
+    return launch_slice_t<false, RB, CB, kSliceWaves, NST, EPI>(a, st)
+    if constexpr (EPI == kPlain) {
+        if (tile == 0) NCM_SLICE(1, 1, 2);
+        if (tile == 1) NCM_SLICE(2, 1, 1);
+    }
+    switch (tile) {
+        case 2: NCM_SLICE(1, 2, 1);
+        case 3: NCM_SLICE(2, 2, 1);
+        case 4: NCM_SLICE(3, 2, 1);
+        case 5: NCM_SLICE(1, 4, 1);
+        case 6: NCM_SLICE(4, 2, 1);
+        case 7: NCM_SLICE(2, 4, 1);
+        case 8: NCM_SLICE(3, 4, 1);
+        case 9: NCM_SLICE(4, 4, 1);
+        case 10: NCM_SLICE(5, 4, 1);
+        default: return hipErrorInvalidValue;
+    }
+#undef NCM_SLICE
+}
+
+}  // namespace
+
+// Where this kernel takes a product, from measurements of both kernels over
+// M = 1 .. 1024 and the projections of the 135M to 8B checkpoints (weights
+// rotated so that they come from HBM). A round of 128 x 128 tiles costs 16 in
+// tile_cost's units, so at cost 13 the small tiles still win: 2048 x 2048
+// with 17 / 128 / 512 rows 17 / 21 / 21 -> 5.6 / 7.4 / 12.2 us, 2048 x 8192
+// with 77 / 203 / 512 rows 58 / 58 / 63 -> 16 / 21 / 31 us; at 14 and above
+// they lose (203 rows, 6144 x 1024: 13.4 -> 14.7 us). With up to 64 rows one row
+// tile covers M, every weight is read once and the weight stream is the
+// bound at any N: 64 rows, 128256 x 2048 162 -> 139 us, 28672 x 4096 55.9 ->
+// 54.8 us; from 65 rows on a wide N would be read twice (77 rows, 28672 x 4096:
+// 54 -> 61 us).
+bool linear_slice_fits(int64_t M, int64_t N, int64_t K) {
+    if (M <= 0 || N <= 0 || K <= 0 || K > (int64_t)1 << 21) return false;
+    int tile;
+    return M <= 64 || best_tile(M, N, false, &tile) <= 13;
+}
+
+hipError_t launch_linear_slice(const uint16_t* x, const uint16_t* w, const uint16_t* bias,
+                               const float* residual, void* y, int64_t M, int64_t K, int64_t N,
+                               int out_mode, hipStream_t st) {
+    SliceArgs a{};
+    a.x = x; a.w = w; a.bias = bias; a.residual = residual; a.y = y;
+    a.M = M; a.K = K; a.N = N;
+    a.out_mode = out_mode;
+    int tile = -1;
+    best_tile(M, N, false, &tile);
+    return launch_slice<kPlain>(tile, a, st);
+}
+
+hipError_t launch_linear_slice_swiglu(const uint16_t* x, const uint16_t* w, const uint16_t* bias,
+                               uint16_t* y, int64_t M, int64_t K, int64_t N2, hipStream_t st) {
+    SliceArgs a{};
+    a.x = x; a.w = w; a.bias = bias; a.y = y;
+    a.M = M; a.K = K; a.N = N2;
+    int tile = -1;
+    best_tile(M, N2, true, &tile);
+    return launch_slice<kSwiGLU>(tile, a, st);
+}
+
+hipError_t launch_linear_slice_rope64(const uint16_t* x, const uint16_t* w, const uint16_t* bias,
+                               uint16_t* y, int64_t M, int64_t K, int64_t N, int64_t rot_cols,
+                               int64_t seq_len, const float* cosine, const float* sine,
+                               hipStream_t st) {
+    SliceArgs a{};
+    a.x = x; a.w = w; a.bias = bias; a.y = y;
+    a.M = M; a.K = K; a.N = N;
+    a.cosine = cosine; a.sine = sine; a.seq_len = seq_len; a.rot_cols = rot_cols;
+    int tile = -1;
+    best_tile(M, N, true, &tile);
+    return launch_slice<kRope>(tile, a, st);
+}
+
+}  // namespace ncm
