@@ -8,7 +8,11 @@
 //   n    = rms_norm(h, post_attention_norm)
 //   a    = silu(n W_gate^T (+ b)) * (n W_up^T (+ b))         (root.zig:255-261)
 //   h    = h + (a W_down^T (+ b))
-// then logits = rms_norm(h, final_norm) W_head^T. The projections run on the
+// then logits = rms_norm(h, final_norm) W_head^T. Where the few-row kernel
+// (linear_slice.hip) takes a product, q|k|v run as one with the rotation of
+// 64-wide heads, gate|up as one with the activation, and o and down with the
+// residual add, the same values bit for bit (a traced stage runs apart).
+// The projections run on the
 // fp32 MFMA (launch_linear_f32: every product exact, the sums in the matrix
 // core's order instead of the reference's increasing k); the bias is added
 // after the product, as the reference's project does. The attention sums
@@ -279,10 +283,35 @@ hipError_t launch_add_f32(float* y, const float* a, int64_t rows, int64_t n, int
 // y [rows, n] = x [rows, k] w^T (+ bias), f32.
 hipError_t project_f32(const float* x, const float* w, const float* bias, float* y, int64_t rows,
                        int64_t k, int64_t n, hipStream_t st) {
+    if (linear_slice_f32_fits(rows, n, k)) {
+        LinearF32 l{};
+        l.x = x; l.w = w; l.bias = bias; l.y = y;
+        l.M = rows; l.K = k; l.N = n;
+        return launch_linear_slice_f32(l, st);
+    }
     NCM_TRY(launch_linear_f32(x, w, y, rows, k, n, st));
     if (bias) NCM_TRY(launch_add_f32(y, bias, rows, n, 1, st));
     return hipSuccess;
 }
+
+namespace {
+
+// hidden [rows, n] += x [rows, k] w^T (+ bias). traced: the product itself is
+// left in proj [rows, n] (scratch otherwise).
+hipError_t project_residual_f32(const float* x, const float* w, const float* bias, float* hidden,
+                                float* proj, bool traced, int64_t rows, int64_t k, int64_t n,
+                                hipStream_t st) {
+    if (!traced && linear_slice_f32_fits(rows, n, k)) {
+        LinearF32 l{};
+        l.x = x; l.w = w; l.bias = bias; l.residual = hidden; l.y = hidden;
+        l.M = rows; l.K = k; l.N = n;
+        return launch_linear_slice_f32(l, st);
+    }
+    NCM_TRY(project_f32(x, w, bias, proj, rows, k, n, st));
+    return launch_add_f32(hidden, proj, rows, n, rows, st);
+}
+
+}  // namespace
 
 hipError_t run_layers_f32(const LayerStackF32& a, hipStream_t st) {
     const ncm_decoder_shape_t& s = *a.shape;
@@ -299,43 +328,66 @@ hipError_t run_layers_f32(const LayerStackF32& a, hipStream_t st) {
                                      st));
         if (L.input_norm_bias) NCM_TRY(launch_add_f32(normed, L.input_norm_bias, T, H, 1, st));
         NCM_TRY(trace_copy(tr.input_norm, l, normed, T, H, st));
-        const float* wq = L.qkv_weight;
-        const float* wk = wq + q_w * H;
-        const float* wv = wk + kv_w * H;
         const float* bq = L.qkv_bias;
-        NCM_TRY(project_f32(normed, wq, bq, q, T, H, q_w, st));
-        NCM_TRY(project_f32(normed, wk, bq ? bq + q_w : nullptr, k, T, H, kv_w, st));
-        NCM_TRY(project_f32(normed, wv, bq ? bq + q_w + kv_w : nullptr, v, T, H, kv_w, st));
+        const int64_t rot = q_w + kv_w, qkv_w = rot + kv_w;
+        if (linear_slice_f32_fits(T, qkv_w, H)) {
+            // One product over the concatenated rows, split into q, k and v as
+            // it is stored; 64-wide heads are rotated on the way.
+            const bool rope = hd == 64 && !L.q_norm;
+            LinearF32 m{};
+            m.x = normed; m.w = L.qkv_weight; m.bias = bq; m.y = q;
+            m.M = T; m.K = H; m.N = qkv_w;
+            m.y1 = k; m.y2 = v; m.n1 = q_w; m.n2 = rot;
+            if (rope) {
+                m.cosine = a.cosine; m.sine = a.sine;
+                m.seq_len = a.seq; m.rot_cols = rot;
+            }
+            NCM_TRY(launch_linear_slice_f32(m, st));
+        } else {
+            const float* wk = L.qkv_weight + q_w * H;
+            const float* wv = wk + kv_w * H;
+            NCM_TRY(project_f32(normed, L.qkv_weight, bq, q, T, H, q_w, st));
+            NCM_TRY(project_f32(normed, wk, bq ? bq + q_w : nullptr, k, T, H, kv_w, st));
+            NCM_TRY(project_f32(normed, wv, bq ? bq + rot : nullptr, v, T, H, kv_w, st));
+        }
         if (L.q_norm) {  // QK-norm (f32 rms_norm of every head) before the rotation
             NCM_TRY(launch_rms_norm_rows(q, L.q_norm, q, T * s.q_heads, hd, s.rms_eps,
                                          NCM_OUT_F32, st));
             NCM_TRY(launch_rms_norm_rows(k, L.k_norm, k, T * s.kv_heads, hd, s.rms_eps,
                                          NCM_OUT_F32, st));
         }
-        NCM_TRY(launch_rope_rotate_f32(q, T, q_w, s.q_heads, hd, a.seq, a.cosine, a.sine, st));
-        NCM_TRY(launch_rope_rotate_f32(k, T, kv_w, s.kv_heads, hd, a.seq, a.cosine, a.sine, st));
+        if (hd != 64 || L.q_norm || !linear_slice_f32_fits(T, qkv_w, H)) {
+            NCM_TRY(launch_rope_rotate_f32(q, T, q_w, s.q_heads, hd, a.seq, a.cosine, a.sine, st));
+            NCM_TRY(launch_rope_rotate_f32(k, T, kv_w, s.kv_heads, hd, a.seq, a.cosine, a.sine,
+                                           st));
+        }
         NCM_TRY(launch_attention_f32(q, k, v, ctx, a.batch, a.seq, s.q_heads, s.kv_heads, hd, q_w,
                                      kv_w, q_w, a.seg_lo ? 0 : s.window, a.prefix, a.seg_lo,
                                      a.seg_hi, a.pad, st));
         NCM_TRY(trace_copy(tr.attention_context, l, ctx, T, q_w, st));
-        NCM_TRY(project_f32(ctx, L.o_weight, L.o_bias, proj, T, q_w, H, st));
+        NCM_TRY(project_residual_f32(ctx, L.o_weight, L.o_bias, hidden, proj, tr.attention_output,
+                                     T, q_w, H, st));
         NCM_TRY(trace_copy(tr.attention_output, l, proj, T, H, st));
-        NCM_TRY(launch_add_f32(hidden, proj, T, H, T, st));
         NCM_TRY(trace_copy(tr.attention_residual, l, hidden, T, H, st));
         NCM_TRY(launch_rms_norm_rows(hidden, L.post_attention_norm, normed, T, H, s.rms_eps,
                                      NCM_OUT_F32, st));
         if (L.post_attention_norm_bias)
             NCM_TRY(launch_add_f32(normed, L.post_attention_norm_bias, T, H, 1, st));
         NCM_TRY(trace_copy(tr.post_attention_norm, l, normed, T, H, st));
-        NCM_TRY(project_f32(normed, L.gate_weight, L.gate_bias, gate, T, H, I, st));
-        NCM_TRY(trace_copy(tr.gate_projection, l, gate, T, I, st));
-        NCM_TRY(project_f32(normed, L.up_weight, L.up_bias, up, T, H, I, st));
-        NCM_TRY(trace_copy(tr.up_projection, l, up, T, I, st));
-        NCM_TRY(launch_silu_mul(gate, up, gate, T * I, NCM_OUT_F32, st));
+        if (!tr.gate_projection && !tr.up_projection && linear_slice_f32_fits(T, I, H)) {
+            NCM_TRY(launch_linear_slice_swiglu_f32(normed, L.gate_weight, L.up_weight,
+                                                   L.gate_bias, L.up_bias, gate, T, H, I, st));
+        } else {
+            NCM_TRY(project_f32(normed, L.gate_weight, L.gate_bias, gate, T, H, I, st));
+            NCM_TRY(trace_copy(tr.gate_projection, l, gate, T, I, st));
+            NCM_TRY(project_f32(normed, L.up_weight, L.up_bias, up, T, H, I, st));
+            NCM_TRY(trace_copy(tr.up_projection, l, up, T, I, st));
+            NCM_TRY(launch_silu_mul(gate, up, gate, T * I, NCM_OUT_F32, st));
+        }
         NCM_TRY(trace_copy(tr.gate_up_product, l, gate, T, I, st));
-        NCM_TRY(project_f32(gate, L.down_weight, L.down_bias, proj, T, I, H, st));
+        NCM_TRY(project_residual_f32(gate, L.down_weight, L.down_bias, hidden, proj,
+                                     tr.mlp_output, T, I, H, st));
         NCM_TRY(trace_copy(tr.mlp_output, l, proj, T, H, st));
-        NCM_TRY(launch_add_f32(hidden, proj, T, H, T, st));
         NCM_TRY(trace_copy(tr.block_output, l, hidden, T, H, st));
     }
     return hipSuccess;

@@ -69,6 +69,34 @@ hipError_t launch_linear_slice_rope64(const uint16_t* x, const uint16_t* w, cons
                                       int64_t rot_cols, int64_t seq_len, const float* cosine,
                                       const float* sine, hipStream_t stream);
 
+// The fp32 K-sliced kernel: y = x w^T (+ bias) (+ residual), all fp32, K % 4
+// == 0, 16-byte aligned x and w. Optional (null / 0 where unused): columns
+// n1 .. n2 - 1 to y1 and n2 .. N - 1 to y2 (each row-major with its own
+// width; then no residual); the rotation of 64-wide heads in columns
+// [0, rot_cols) with table row (row % seq_len) (N and rot_cols multiples of
+// 64; then no residual).
+struct LinearF32 {
+    const float* x;
+    const float* w;
+    const float* bias;
+    const float* residual;  // [M, N], may be y
+    float* y;
+    int64_t M, K, N;
+    float* y1;
+    float* y2;
+    int64_t n1, n2;
+    const float* cosine;
+    const float* sine;
+    int64_t seq_len, rot_cols;
+};
+// Whether it takes an M x N x K product (launch_linear_f32 asks).
+bool linear_slice_f32_fits(int64_t M, int64_t N, int64_t K);
+hipError_t launch_linear_slice_f32(const LinearF32& l, hipStream_t stream);
+// y [M, N] = silu(x gate^T (+ gate_bias)) * (x up^T (+ up_bias)); gate, up [N, K].
+hipError_t launch_linear_slice_swiglu_f32(const float* x, const float* gate, const float* up,
+                                          const float* gate_bias, const float* up_bias, float* y,
+                                          int64_t M, int64_t K, int64_t N, hipStream_t stream);
+
 // fp32 operands, fp32 output; K % 4 == 0, 16-byte aligned x and w.
 hipError_t launch_linear_f32(const float* x, const float* w, float* y, int64_t M, int64_t K,
                              int64_t N, hipStream_t stream);

@@ -337,6 +337,12 @@ hipError_t launch_linear_residual(const uint16_t* x, const uint16_t* w, const ui
 
 hipError_t launch_linear_f32(const float* x, const float* w, float* y, int64_t M, int64_t K,
                              int64_t N, hipStream_t stream) {
+    if (linear_slice_f32_fits(M, N, K)) {
+        LinearF32 l{};
+        l.x = x; l.w = w; l.y = y;
+        l.M = M; l.K = K; l.N = N;
+        return launch_linear_slice_f32(l, stream);
+    }
     return launch_linear_t<LinF32, NCM_OUT_F32, false>(x, w, nullptr, y, M, K, N, stream);
 }
 

@@ -44,6 +44,15 @@ struct SliceArgs {
     void* y;
     int64_t M, K, N;  // N: weight rows
     int out_mode, tiles_m;
+    // fp32 only: the bias; SwiGLU's up rows and bias (w and bias32: gate);
+    // columns n1 .. n2 - 1 go to y1 and n2 .. N - 1 to y2 (rows of their own
+    // width, n1 = 0: all to y).
+    const float* bias32;
+    const float* w2;
+    const float* bias2;
+    float* y1;
+    float* y2;
+    int64_t n1, n2;
     // RoPE: tables [seq_len, 64], columns [0, rot_cols) rotated.
     const float* cosine;
     const float* sine;
@@ -87,14 +96,23 @@ __global__ __launch_bounds__(64 * NW) void linear_slice_kernel(SliceArgs a) {
     // First weight row. The paired epilogues (gate and up rows, or the two
     // halves of a head) need rows c and c + 32 of a 64-row group together:
     // CB = 4 takes the group, CB = 2 its rows s .. s + 15 and s + 32 .. s + 47.
-    const int64_t n0 = EPI == kPlain || CB == 4 ? (int64_t)tn * 16 * CB
-                                                : (int64_t)(tn >> 1) * 64 + (tn & 1) * 16;
-    constexpr int BSTEP = EPI != kPlain && CB == 2 ? 32 : 16;  // rows between column blocks
+    // (fp32 SwiGLU: the same CB / 2 blocks of rows from each of two matrices.)
+    constexpr bool TWO_W = F32 && EPI == kSwiGLU;
+    constexpr int HB = CB > 1 ? CB / 2 : 1;
+    const int64_t n0 = TWO_W ? (int64_t)tn * 16 * HB
+                       : EPI == kPlain || CB == 4
+                           ? (int64_t)tn * 16 * CB
+                           : (int64_t)(tn >> 1) * 64 + (tn & 1) * 16;
+    // Rows between column blocks.
+    constexpr int BSTEP = !TWO_W && EPI != kPlain && CB == 2 ? 32 : 16;
     const int64_t K = a.K;
     const __amdgpu_buffer_rsrc_t rsx =
         make_rsrc((const char*)a.x + m0 * K * ESZ, operand_bytes(a.M, m0, K, ESZ));
     const __amdgpu_buffer_rsrc_t rsw =
         make_rsrc((const char*)a.w + n0 * K * ESZ, operand_bytes(a.N, n0, K, ESZ));
+    const __amdgpu_buffer_rsrc_t rsw2 =
+        make_rsrc((const char*)(TWO_W ? a.w2 : a.w) + n0 * K * ESZ,
+                  operand_bytes(a.N, n0, K, ESZ));
 
     // Load instruction p fills LDS rows 8 p .. 8 p + 7 (x rows, then weight
     // rows), lane l row l / 8, chunk slot l % 8; the swizzle term depends on
@@ -113,9 +131,10 @@ __global__ __launch_bounds__(64 * NW) void linear_slice_kernel(SliceArgs a) {
         for (int p = 0; p < S::ND; ++p) {
             const bool is_x = p < 2 * RB;
             const int q = is_x ? p : p - 2 * RB;
-            const int row = is_x ? 8 * q : (q >> 1) * BSTEP + 8 * (q & 1);
+            const int cb = TWO_W ? (q >> 1) % HB : q >> 1;
+            const int row = is_x ? 8 * q : cb * BSTEP + 8 * (q & 1);
             __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                is_x ? rsx : rsw,
+                is_x ? rsx : (TWO_W && q >= 2 * HB ? rsw2 : rsw),
                 (__attribute__((address_space(3))) void*)(stage + p * 1024), 16,
                 (p & 1 ? v1 : v0) + (uint32_t)row * rowb, 0, 0, 0);
         }
@@ -198,7 +217,16 @@ __global__ __launch_bounds__(64 * NW) void linear_slice_kernel(SliceArgs a) {
         return s;
     };
     auto bias_of = [&](int64_t n) {
+        if (F32) return a.bias32 ? a.bias32[n] : 0.0f;
         return a.bias ? __uint_as_float((uint32_t)a.bias[n] << 16) : 0.0f;
+    };
+    const bool has_bias = F32 ? a.bias32 != nullptr : a.bias != nullptr;
+    // fp32 output element (m, n) under the column split.
+    auto out32 = [&](int64_t m, int64_t n) -> float* {
+        if (a.n1 == 0) return (float*)a.y + m * a.N + n;
+        if (n < a.n1) return (float*)a.y + m * a.n1 + n;
+        if (n < a.n2) return a.y1 + m * (a.n2 - a.n1) + n - a.n1;
+        return a.y2 + m * (a.N - a.n2) + n - a.n2;
     };
 
     if constexpr (EPI == kPlain) {
@@ -212,8 +240,10 @@ __global__ __launch_bounds__(64 * NW) void linear_slice_kernel(SliceArgs a) {
                 const int64_t m = m0 + 16 * (b / CB) + 4 * grp + j;
                 if (m >= a.M) continue;
                 const int64_t off = m * a.N + n;
-                const float f = a.bias ? v[j] + bv : v[j];
-                if (a.out_mode == NCM_OUT_F32) {
+                const float f = has_bias ? v[j] + bv : v[j];
+                if constexpr (F32) {
+                    *out32(m, n) = a.residual ? a.residual[off] + f : f;
+                } else if (a.out_mode == NCM_OUT_F32) {
                     ((float*)a.y)[off] = a.residual ? a.residual[off] + f : f;
                 } else {
                     uint32_t bits = bf16_bits_rne(flush_subnormal(f));
@@ -229,12 +259,49 @@ __global__ __launch_bounds__(64 * NW) void linear_slice_kernel(SliceArgs a) {
         return;
     }
     // Pairs: column blocks cb and cb + CB / 2, 32 weight rows apart.
-    constexpr int HB = CB > 1 ? CB / 2 : 1;
     for (int b = wave; b < RB * HB; b += NW) {
         const int rb = b / HB, cb = b % HB;
         const f32x4_t va = sum(rb * CB + cb), vb = sum(rb * CB + cb + HB);
-        const int64_t na = n0 + 16 * cb + r16;  // N % 64 == 0: the pair is in range
+        const int64_t na = n0 + 16 * cb + r16;
+        if constexpr (TWO_W) {
+            // silu(g) * u, unrounded (root.zig:255-261, src/decoder.zig:210-211).
+            if (na >= a.N) continue;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int64_t m = m0 + 16 * rb + 4 * grp + j;
+                if (m >= a.M) continue;
+                const float g = a.bias32 ? va[j] + a.bias32[na] : va[j];
+                const float u = a.bias2 ? vb[j] + a.bias2[na] : vb[j];
+                const float sigmoid = 1.0f / (1.0f + expf(-g));
+                const float act = g * sigmoid;
+                ((float*)a.y)[m * a.N + na] = act * u;
+            }
+            continue;
+        }
+        // N % 64 == 0: the pair is in range.
         const float ba = bias_of(na), bb = bias_of(na + 32);
+        if constexpr (F32 && EPI == kRope) {
+            // rotate_head in f32 mode (root.zig:615-634).
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int64_t m = m0 + 16 * rb + 4 * grp + j;
+                if (m >= a.M) continue;
+                float first = has_bias ? va[j] + ba : va[j];
+                float second = has_bias ? vb[j] + bb : vb[j];
+                if (na < a.rot_cols) {
+                    const int64_t t = (m % a.seq_len) * 64 + (na & 63);
+                    const float left = first * a.cosine[t];
+                    const float right = -second * a.sine[t];
+                    const float right2 = first * a.sine[t + 32];
+                    const float left2 = second * a.cosine[t + 32];
+                    first = left + right;
+                    second = left2 + right2;
+                }
+                *out32(m, na) = first;
+                *out32(m, na + 32) = second;
+            }
+            continue;
+        }
         uint16_t* y = (uint16_t*)a.y;
 #pragma unroll
         for (int j = 0; j < 4; j += 2) {
@@ -281,7 +348,8 @@ hipError_t launch_slice_t(SliceArgs a, hipStream_t st) {
         (const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, S::LDS);
     if (attr != hipSuccess) return attr;
     a.tiles_m = (int)((a.M + 16 * RB - 1) / (16 * RB));
-    const int64_t blocks = a.tiles_m * ((a.N + 16 * CB - 1) / (16 * CB));
+    constexpr int COLS = F32 && EPI == kSwiGLU ? 8 * CB : 16 * CB;  // of N per workgroup
+    const int64_t blocks = a.tiles_m * ((a.N + COLS - 1) / COLS);
     hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(64 * NW), S::LDS, st, a);
     return hipGetLastError();
 }
@@ -327,10 +395,10 @@ int64_t best_tile(int64_t M, int64_t N, bool paired, int* tile) {
     return best;
 }
 
-template <int EPI>
+template <int EPI, bool F32 = false>
 hipError_t launch_slice(int tile, const SliceArgs& a, hipStream_t st) {
 #define NCM_SLICE(RB, CB, NST) \
-    return launch_slice_t<false, RB, CB, kSliceWaves, NST, EPI>(a, st)
+    return launch_slice_t<F32, RB, CB, kSliceWaves, NST, EPI>(a, st)
     if constexpr (EPI == kPlain) {
         if (tile == 0) NCM_SLICE(1, 1, 2);
         if (tile == 1) NCM_SLICE(2, 1, 1);
@@ -348,6 +416,33 @@ hipError_t launch_slice(int tile, const SliceArgs& a, hipStream_t st) {
         default: return hipErrorInvalidValue;
     }
 #undef NCM_SLICE
+}
+
+// fp32: the matrix core is the bound (1/16 of the bf16 rate), so a tile is
+// priced in time: rounds of the CUs times the workgroup's MFMAs (0.22 us per
+// block of 16 x 16 outputs and iteration of its eight wavefronts) plus what
+// starting, summing and storing it takes. Fitted to M = 1 .. 600 on the 135M and
+// 0.5B checkpoints' projections, within 20% where the weight stream is not the
+// bound (200 rows, 576 x 576: 4.9 us; 300 rows, 4864 x 896: 35 us).
+double f32_tile_us(const Tile& s, int64_t M, int64_t N, int64_t K) {
+    const int64_t tiles =
+        ((M + 16 * s.rb - 1) / (16 * s.rb)) * ((N + 16 * s.cb - 1) / (16 * s.cb));
+    const int64_t iters = ((K + 31) / 32 + kSliceWaves - 1) / kSliceWaves;
+    const int blocks = s.rb * s.cb;
+    return (double)((tiles + 255) / 256) * (0.22 * blocks * iters + 1.3 + 0.3 * blocks);
+}
+
+double best_tile_f32(int64_t M, int64_t N, int64_t K, bool paired, int* tile) {
+    double best = 1e300;
+    for (int t = 0; t < kTileCount; ++t) {
+        if (paired && kTiles[t].cb < 2) continue;
+        const double us = f32_tile_us(kTiles[t], M, N, K);
+        if (us < best) {
+            best = us;
+            *tile = t;
+        }
+    }
+    return best;
 }
 
 }  // namespace
@@ -402,6 +497,40 @@ hipError_t launch_linear_slice_rope64(const uint16_t* x, const uint16_t* w, cons
     int tile = -1;
     best_tile(M, N, true, &tile);
     return launch_slice<kRope>(tile, a, st);
+}
+
+// The 128 x 128 fp32 tiles take 2.03 us per 32-element K tile and round of the
+// CUs (130 us for anything up to 256 tiles at K = 2048).
+bool linear_slice_f32_fits(int64_t M, int64_t N, int64_t K) {
+    if (M <= 0 || N <= 0 || K <= 0 || K > (int64_t)1 << 20) return false;
+    const int64_t big = ((M + 127) / 128) * ((N + 127) / 128);
+    const double big_us = (double)((big + 255) / 256) * (2.03 * ((K + 31) / 32) + 3.5);
+    int tile;
+    return best_tile_f32(M, N, K, false, &tile) < big_us;
+}
+
+hipError_t launch_linear_slice_f32(const LinearF32& l, hipStream_t st) {
+    SliceArgs a{};
+    a.x = l.x; a.w = l.w; a.bias32 = l.bias; a.residual = l.residual; a.y = l.y;
+    a.M = l.M; a.K = l.K; a.N = l.N;
+    a.y1 = l.y1; a.y2 = l.y2; a.n1 = l.n1; a.n2 = l.n2;
+    a.cosine = l.cosine; a.sine = l.sine; a.seq_len = l.seq_len; a.rot_cols = l.rot_cols;
+    const bool rope = l.cosine != nullptr;
+    if (rope && (l.N % 64 || l.rot_cols % 64 || l.seq_len <= 0)) return hipErrorInvalidValue;
+    int tile = -1;
+    best_tile_f32(l.M, l.N, l.K, rope, &tile);
+    return rope ? launch_slice<kRope, true>(tile, a, st) : launch_slice<kPlain, true>(tile, a, st);
+}
+
+hipError_t launch_linear_slice_swiglu_f32(const float* x, const float* gate, const float* up,
+                                          const float* gate_bias, const float* up_bias, float* y,
+                                          int64_t M, int64_t K, int64_t N, hipStream_t st) {
+    SliceArgs a{};
+    a.x = x; a.w = gate; a.w2 = up; a.bias32 = gate_bias; a.bias2 = up_bias; a.y = y;
+    a.M = M; a.K = K; a.N = N;
+    int tile = -1;
+    best_tile_f32(M, 2 * N, K, true, &tile);
+    return launch_slice<kSwiGLU, true>(tile, a, st);
 }
 
 }  // namespace ncm

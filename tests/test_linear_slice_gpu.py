@@ -81,3 +81,62 @@ def test_slice_fused_epilogues(ncm, oracle, cuda, m, k, inter, bias):
         kernels.rope_rotate(ref[:, :rot], rot // 64, 64, seq, cd, sd)
     got = kernels.linear_bf16_rope64(x, w, rot, seq, cd, sd, bias=b)
     assert torch.equal(got.view(torch.int16), ref.view(torch.int16))
+
+
+# K below, at and past one round of the wavefronts' 32-element tiles; N of one
+# and of several rounds; the last one past the small tiles' range.
+@pytest.mark.parametrize("m,k,n", [(1, 4, 1), (17, 576, 960), (33, 260, 1153), (77, 4864, 896),
+                                   (200, 576, 577), (300, 1000, 4864), (600, 36, 130),
+                                   (130, 896, 20000)])
+def test_slice_f32(ncm, cuda, m, k, n):
+    import torch
+    from ncmorph_amd import kernels
+
+    print(f"slice f32 m={m} k={k} n={n}", flush=True)
+    rng = np.random.default_rng(m + k + n)
+    x = torch.from_numpy(rng.standard_normal((m, k)).astype(np.float32)).to(cuda)
+    w = torch.from_numpy(rng.standard_normal((n, k)).astype(np.float32)).to(cuda)
+    y = kernels.linear_f32(x, w)
+    ref = x.double() @ w.double().t()
+    bound = (x.double().abs() @ w.double().abs().t()) * (k + 1) * 2.0**-24
+    assert bool(((y.double() - ref).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("hidden,inter,hq,hkv,hd,t,biases", [(128, 256, 4, 2, 64, 37, True),
+                                                             (576, 1536, 9, 3, 64, 77, False),
+                                                             (96, 68, 3, 1, 32, 20, True)])
+def test_f32_decoder_fused_equals_traced(ncm, oracle, cuda, hidden, inter, hq, hkv, hd, t,
+                                         biases):
+    """Without a trace the f32 layers run one q|k|v product with the rotation,
+    gate|up with the activation and the residual adds inside the products; with
+    every stage traced those run apart. The same bits."""
+    import torch
+    from ncmorph_amd import decoder
+
+    print(f"f32 decoder fused hidden={hidden} hd={hd} t={t}", flush=True)
+    g = torch.Generator(device=cuda).manual_seed(hidden + t)
+
+    def r(*shape, std=0.1):
+        return torch.randn(*shape, generator=g, device=cuda) * std
+
+    qkv = (hq + 2 * hkv) * hd
+    layers = []
+    for _ in range(2):
+        layer = {"input_norm": 1 + r(hidden), "qkv_weight": r(qkv, hidden),
+                 "o_weight": r(hidden, hq * hd), "post_attention_norm": 1 + r(hidden),
+                 "gate_weight": r(inter, hidden), "up_weight": r(inter, hidden),
+                 "down_weight": r(hidden, inter)}
+        if biases:
+            layer.update(qkv_bias=r(qkv), o_bias=r(hidden), gate_bias=r(inter),
+                         up_bias=r(inter), down_bias=r(hidden))
+        layers.append(layer)
+    spec = decoder.DecoderSpec(hidden=hidden, intermediate=inter, vocab=200, q_heads=hq,
+                               kv_heads=hkv, head_dim=hd, layers=2, rope_theta=10000.0)
+    w = decoder.DecoderWeights(embed=r(200, hidden), final_norm=1 + r(hidden), layers=layers,
+                               mode="f32")
+    cos, sin = oracle.rope_tables(oracle.rope_default_frequencies(hd, 10000.0), t)
+    tables = torch.from_numpy(cos).to(cuda), torch.from_numpy(sin).to(cuda)
+    ids = np.random.default_rng(t).integers(0, 200, (2, t))
+    plain = decoder.forward_f32(spec, w, ids, *tables)
+    traced, _ = decoder.forward_f32(spec, w, ids, *tables, trace=True)
+    assert torch.equal(plain, traced)
