@@ -90,127 +90,284 @@ hipError_t launch_rope_rotate_f32(float* x, int64_t rows, int64_t row_stride, in
 }
 
 constexpr int kAttnF32MaxHd = 256;
+constexpr int kAttnQ = 8;          // queries (wavefronts) per workgroup
+constexpr int kAttnPanel = 2048;   // keys whose scores a workgroup keeps in LDS
 
-// f32-mode attention of one (sequence, query, head) per wavefront, four
-// heads per workgroup: grid (seq_len, ceil(q_heads / 4), batch). Allowed
-// keys, in increasing order: causal, [k_lo, query] (optionally windowed); or
-// with the level mask (seg_lo set), the prefix keys 0 .. prefix-1 whose pad
-// bit is clear, then [seg_lo[q], seg_hi[q]) (at or after the prefix). They
-// are walked 64 per chunk, one per lane, three times: the maximum score; the
-// softmax sum, added in key order (every lane adds the chunk's exponentials
-// in lane order); then p = exp(s - max) / sum and the context, lane =
-// dimension, adding p_k v_k in key order. A score is the dot product in
-// dimension order, then times 1 / sqrt(hd). Masked keys (probability 0) add
-// nothing, as in the reference unless V holds an infinity or NaN there; a
-// query with no allowed key gets a zero context (root.zig:563-565).
-__global__ __launch_bounds__(256) void attention_f32_kernel(
+// f32-mode attention: a workgroup takes eight queries of one (sequence, head),
+// one per wavefront, and stages KC keys (then their values) at a time in LDS
+// for all of them, the next ones on their way in registers. A score is the dot product in dimension order (lane = key),
+// then times 1 / sqrt(hd); the softmax sum runs in key order, and so does
+// every context element (lane = dimension): the reference's orders, so only
+// exp differs from it (device expf). The scores of up to kAttnPanel keys stay
+// in LDS and are formed once; past that they are formed again, panel by
+// panel, for the sum and for the context. Allowed keys, in increasing order:
+// causal, [query - window + 1, query]; or with the level mask (seg_lo set),
+// the prefix keys whose pad bit is clear, then [seg_lo[q], seg_hi[q]) (at or
+// after the prefix). Masked keys (probability 0) add nothing, as in the
+// reference unless V holds an infinity or NaN there; a query with no allowed
+// key gets a zero context (root.zig:563-565).
+//
+// What bounds it at a 200-token prompt of 9 heads (225 workgroups): the chains
+// of one wavefront (64 adds a score, one add a key in the sum and in the
+// context), not memory. One wavefront per (query, head) that walked the keys
+// three times, reading every K row from the caches by itself, took 90 us a
+// layer there; this takes 17.
+
+// Orders LDS accesses of one wavefront's lanes (its LDS operations run in
+// program order; this keeps the compiler from moving them).
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// HS: ceil(hd / 64); KC: 128, or 64 where 128 rows would not fit.
+template <int HS, int KC>
+__global__ __launch_bounds__(64 * kAttnQ) void attention_f32_kernel(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
-    float* __restrict__ out, int64_t T, int q_heads, int group, int hd, int64_t q_stride,
-    int64_t kv_stride, int64_t out_stride, int64_t window, float scale, int64_t prefix,
+    float* __restrict__ out, int64_t T, int group, int hd, int64_t q_stride, int64_t kv_stride,
+    int64_t out_stride, int64_t window, float scale, int64_t prefix,
     const int32_t* __restrict__ seg_lo, const int32_t* __restrict__ seg_hi,
-    const uint64_t* __restrict__ pad) {
+    const uint64_t* __restrict__ pad, int panel) {
+    // [KC][hd + 4] staged K or V rows, [kAttnQ][hd] queries, then
+    // [kAttnQ][panel + 4] scores.
+    extern __shared__ __attribute__((aligned(16))) float smem[];
+    const int ld = hd + 4, sld = panel + 4;
+    float* rows = smem;
+    float* qs = rows + KC * ld;
     const int lane = threadIdx.x & 63;
-    const int h = blockIdx.y * 4 + (threadIdx.x >> 6);
-    if (h >= q_heads) return;
-    const int64_t b = blockIdx.z, qi = blockIdx.x;
-    const int kvh = h / group;
-    const float* qrow = q + (b * T + qi) * q_stride + (int64_t)h * hd;
-    const float* kbase = k + b * T * kv_stride + (int64_t)kvh * hd;
-    const float* vbase = v + b * T * kv_stride + (int64_t)kvh * hd;
-    // q spread over the lanes: dimension d in lane d % 64, slot d / 64.
-    float qv[kAttnF32MaxHd / 64];
-#pragma unroll
-    for (int s = 0; s < kAttnF32MaxHd / 64; ++s) {
-        const int d = s * 64 + lane;
-        qv[s] = d < hd ? qrow[d] : 0.0f;
-    }
-    // Key j of the walk (j in [0, nkeys)) and whether it is allowed.
-    int64_t nkeys, k_lo = 0, lo = 0, P = 0;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    float* sc = qs + kAttnQ * hd + wave * sld;
+    const int h = blockIdx.y;
+    const int64_t b = blockIdx.z;
+    // The last queries (the most keys under a causal mask) first.
+    const int64_t q0 = (int64_t)(gridDim.x - 1 - blockIdx.x) * kAttnQ;
+    const int64_t qi = q0 + wave;
+    const bool live = qi < T;
+    const float* qrow = q + (b * T + (live ? qi : q0)) * q_stride + (int64_t)h * hd;
+    const float* kbase = k + b * T * kv_stride + (int64_t)(h / group) * hd;
+    const float* vbase = v + b * T * kv_stride + (int64_t)(h / group) * hd;
+    for (int d = lane; d < hd; d += 64) qs[wave * hd + d] = qrow[d];
+
+    // The walk of the workgroup: keys 0 .. P - 1, then base .. end - 1, the
+    // union of its queries' ranges; this query's own range is [lo, hi).
+    const int64_t P = seg_lo ? prefix : 0;
+    int64_t base, end, lo, hi;
     if (seg_lo) {
-        P = prefix;
-        lo = seg_lo[b * T + qi];
-        const int64_t hi = seg_hi[b * T + qi];
-        nkeys = P + (hi > lo ? hi - lo : 0);
-    } else {
-        k_lo = window > 0 ? qi - window + 1 : 0;
-        if (k_lo < 0) k_lo = 0;
-        nkeys = qi + 1 - k_lo;
-    }
-    auto key_of = [&](int64_t j) { return seg_lo ? (j < P ? j : lo + (j - P)) : k_lo + j; };
-    auto allowed = [&](int64_t j) {
-        if (j >= nkeys) return false;
-        if (seg_lo && j < P && pad) return ((pad[j >> 6] >> (j & 63)) & 1ull) == 0ull;
-        return true;
-    };
-    // q . k in dimension order (separate multiply and add), then * scale;
-    // the q values come from their lanes, the k row in 16-byte loads.
-    auto score_of = [&](int64_t key) {
-        const float* kr = kbase + key * kv_stride;
-        float s = 0.0f;
-#pragma unroll
-        for (int sl = 0; sl < kAttnF32MaxHd / 64; ++sl) {
-            if (sl * 64 >= hd) break;
-            const uint32_t qbits = __float_as_uint(qv[sl]);
-            const int nd = hd - sl * 64 < 64 ? hd - sl * 64 : 64;
-            for (int j = 0; j < nd; j += 4) {
-                const f32x4_t k4 = *(const f32x4_t*)(kr + sl * 64 + j);
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    s = s + __uint_as_float(__builtin_amdgcn_readlane(qbits, j + e)) * k4[e];
+        base = T;
+        end = 0;
+        lo = hi = 0;
+        for (int i = 0; i < kAttnQ && q0 + i < T; ++i) {
+            const int64_t l = seg_lo[b * T + q0 + i], e = seg_hi[b * T + q0 + i];
+            if (i == wave) {
+                lo = l;
+                hi = e;
+            }
+            if (e > l) {
+                base = l < base ? l : base;
+                end = e > end ? e : end;
             }
         }
-        return s * scale;
+        if (end < base) base = end = P;
+    } else {
+        const int64_t last = q0 + kAttnQ < T ? q0 + kAttnQ : T;
+        base = window > 0 && q0 - window + 1 > 0 ? q0 - window + 1 : 0;
+        end = last;
+        lo = window > 0 && qi - window + 1 > 0 ? qi - window + 1 : 0;
+        hi = qi + 1;
+    }
+    const int64_t nkeys = P + end - base;
+    auto key_of = [&](int64_t j) { return j < P ? j : base + (j - P); };
+    auto allowed = [&](int64_t j) {
+        if (!live || j >= nkeys) return false;
+        if (j < P) return !pad || ((pad[j >> 6] >> (j & 63)) & 1ull) == 0ull;
+        const int64_t key = key_of(j);
+        return key >= lo && key < hi;
     };
-    // Walk 1: the maximum.
+    // Staging: TPR threads a row, thread t % TPR its 16-byte chunks t % TPR,
+    // + TPR, ...
+    constexpr int TPR = 64 * kAttnQ / KC;
+    constexpr int NV = 16 * HS / TPR;
+    const int srow = threadIdx.x / TPR, sch = threadIdx.x % TPR;
+    f32x4_t pre[NV];
+    auto fetch = [&](const float* src, int64_t c0) {
+        const int64_t j = c0 + srow < nkeys ? c0 + srow : nkeys - 1;
+        const float* r = src + key_of(j) * kv_stride;
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+            if (4 * (sch + TPR * i) < hd) pre[i] = *(const f32x4_t*)(r + 4 * (sch + TPR * i));
+    };
+    auto stage = [&]() {
+        __syncthreads();  // every wavefront is past the rows staged before
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+            if (4 * (sch + TPR * i) < hd)
+                *(f32x4_t*)(rows + srow * ld + 4 * (sch + TPR * i)) = pre[i];
+        __syncthreads();
+    };
+    // Scores of keys [p0, p1) into sc (masked: -inf); returns the maximum of
+    // each lane's own keys. The first KC keys are already fetched; the first
+    // values are fetched under the last keys' products.
+    auto scores = [&](int64_t p0, int64_t p1) {
+        float m = -INFINITY;
+        for (int64_t c0 = p0; c0 < p1; c0 += KC) {
+            stage();
+            if (c0 + KC < p1)
+                fetch(kbase, c0 + KC);
+            else
+                fetch(vbase, p0);
+            bool ok[KC / 64];
+            float s[KC / 64];
+#pragma unroll
+            for (int u = 0; u < KC / 64; ++u) {
+                ok[u] = allowed(c0 + 64 * u + lane);
+                s[u] = 0.0f;
+            }
+            const float* kr = rows + lane * ld;
+            const float* qr = qs + wave * hd;
+#pragma unroll 4
+            for (int d = 0; d < hd; d += 4) {
+                const f32x4_t q4 = *(const f32x4_t*)(qr + d);
+#pragma unroll
+                for (int u = 0; u < KC / 64; ++u) {
+                    const f32x4_t k4 = *(const f32x4_t*)(kr + 64 * u * ld + d);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) s[u] = s[u] + q4[e] * k4[e];
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < KC / 64; ++u) {
+                const float t = ok[u] ? s[u] * scale : -INFINITY;
+                sc[c0 - p0 + 64 * u + lane] = t;
+                m = fmaxf(m, t);
+            }
+        }
+        return m;
+    };
+
+    if (nkeys <= 0) {  // the whole workgroup
+        if (live)
+            for (int d = lane; d < hd; d += 64)
+                out[(b * T + qi) * out_stride + (int64_t)h * hd + d] = 0.0f;
+        return;
+    }
+    const bool once = nkeys <= panel;
     float m = -INFINITY;
-    for (int64_t c0 = 0; c0 < nkeys; c0 += 64) {
-        const int64_t j = c0 + lane;
-        const float s = allowed(j) ? score_of(key_of(j)) : -INFINITY;
-        m = fmaxf(m, s);
+    for (int64_t p0 = 0; p0 < nkeys; p0 += panel) {
+        fetch(kbase, p0);
+        m = fmaxf(m, scores(p0, p0 + panel < nkeys ? p0 + panel : nkeys));
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
-    float acc[kAttnF32MaxHd / 64];
-#pragma unroll
-    for (int s = 0; s < kAttnF32MaxHd / 64; ++s) acc[s] = 0.0f;
-    if (m != -INFINITY) {
-        // Walk 2: the sum, in key order.
-        float sum = 0.0f;
-        for (int64_t c0 = 0; c0 < nkeys; c0 += 64) {
-            const int64_t j = c0 + lane;
-            const bool ok = allowed(j);
-            const float e = ok ? expf(score_of(key_of(j)) - m) : 0.0f;
-            const uint64_t okm = __ballot(ok);
-            const int n = (int)(nkeys - c0 < 64 ? nkeys - c0 : 64);
-            for (int jj = 0; jj < n; ++jj)
-                if ((okm >> jj) & 1ull)
-                    sum = sum + __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(e), jj));
+    // The sum, in key order (a masked key adds 0, which changes no bit).
+    float sum = 0.0f;
+    for (int64_t p0 = 0; p0 < nkeys; p0 += panel) {
+        const int64_t p1 = p0 + panel < nkeys ? p0 + panel : nkeys;
+        if (!once) {
+            fetch(kbase, p0);
+            scores(p0, p1);
         }
-        // Walk 3: probabilities and the context, lane = dimension.
-        for (int64_t c0 = 0; c0 < nkeys; c0 += 64) {
-            const int64_t j = c0 + lane;
-            const bool ok = allowed(j);
-            const float p = ok ? expf(score_of(key_of(j)) - m) / sum : 0.0f;
-            const uint64_t okm = __ballot(ok);
-            const int n = (int)(nkeys - c0 < 64 ? nkeys - c0 : 64);
-            for (int jj = 0; jj < n; ++jj) {
-                if (!((okm >> jj) & 1ull)) continue;
-                const float pj = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(p), jj));
-                const float* vr = vbase + key_of(c0 + jj) * kv_stride;
+        const int n = (int)(p1 - p0);
+        wave_lds_fence();
+        for (int j = lane; j < ((n + 63) & ~63); j += 64) {
+            const float s = sc[j];
+            sc[j] = allowed(p0 + j) ? expf(s - m) : 0.0f;
+        }
+        wave_lds_fence();
+#pragma unroll 4
+        for (int j = 0; j < n; j += 4) {  // past n: zeros
+            const f32x4_t e = *(const f32x4_t*)(sc + j);
+            sum = sum + e[0];
+            sum = sum + e[1];
+            sum = sum + e[2];
+            sum = sum + e[3];
+        }
+    }
+    // Probabilities and the context, lane = dimension.
+    float acc[HS];
 #pragma unroll
-                for (int s = 0; s < kAttnF32MaxHd / 64; ++s) {
-                    const int d = s * 64 + lane;
-                    if (d < hd) acc[s] = acc[s] + pj * vr[d];
+    for (int s = 0; s < HS; ++s) acc[s] = 0.0f;
+    for (int64_t p0 = 0; p0 < nkeys; p0 += panel) {
+        const int64_t p1 = p0 + panel < nkeys ? p0 + panel : nkeys;
+        if (!once) {
+            fetch(kbase, p0);
+            scores(p0, p1);
+        }
+        const int n = (int)(p1 - p0);
+        wave_lds_fence();
+        for (int j = lane; j < ((n + 63) & ~63); j += 64) {
+            const float s = sc[j];
+            sc[j] = (once ? s : expf(s - m)) / sum;
+        }
+        for (int64_t c0 = p0; c0 < p1; c0 += 64) {
+            const int half = (int)(c0 - p0) % KC;
+            if (half == 0) {
+                stage();
+                if (c0 + KC < p1) fetch(vbase, c0 + KC);
+            }
+            // No finite maximum: every probability is 0 (root.zig:563-565).
+            uint64_t okm = m == -INFINITY ? 0ull : __ballot(allowed(c0 + lane));
+            const float* pr = sc + (c0 - p0);
+            const float* vr = rows + half * ld + lane;
+            if (okm == ~0ull) {
+#pragma unroll 4
+                for (int j = 0; j < 64; j += 4) {
+                    const f32x4_t p4 = *(const f32x4_t*)(pr + j);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+#pragma unroll
+                        for (int s = 0; s < HS; ++s)
+                            acc[s] = acc[s] + p4[e] * vr[(j + e) * ld + 64 * s];
                 }
+                continue;
+            }
+            // Some keys masked: four at a time, a masked one leaves acc alone.
+            for (int j = 0; j < 64; j += 4) {
+                const uint32_t ok4 = (uint32_t)(okm >> j) & 15u;
+                if (!ok4) continue;
+                const f32x4_t p4 = *(const f32x4_t*)(pr + j);
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int s = 0; s < HS; ++s) {
+                        const float t = acc[s] + p4[e] * vr[(j + e) * ld + 64 * s];
+                        acc[s] = (ok4 >> e) & 1u ? t : acc[s];
+                    }
             }
         }
     }
+    if (!live) return;
     float* orow = out + (b * T + qi) * out_stride + (int64_t)h * hd;
 #pragma unroll
-    for (int s = 0; s < kAttnF32MaxHd / 64; ++s) {
+    for (int s = 0; s < HS; ++s) {
         const int d = s * 64 + lane;
         if (d < hd) orow[d] = acc[s];
     }
+}
+
+template <int HS, int KC>
+hipError_t launch_attention_f32_t(const float* q, const float* k, const float* v, float* out,
+                                  int64_t batch, int64_t T, int q_heads, int kv_heads, int hd,
+                                  int64_t q_stride, int64_t kv_stride, int64_t out_stride,
+                                  int64_t window, int64_t prefix, const int32_t* seg_lo,
+                                  const int32_t* seg_hi, const uint64_t* pad, hipStream_t st) {
+    auto kern = attention_f32_kernel<HS, KC>;
+    // A lane past hd reads up to 64 HS - hd floats beyond its row: the query
+    // and score arrays that follow the staged rows hold them.
+    constexpr int max_hd = 64 * HS;
+    constexpr int max_lds =
+        4 * (KC * (max_hd + 4) + kAttnQ * max_hd + kAttnQ * (kAttnPanel + 4));
+    static_assert(max_lds <= 160 * 1024, "LDS budget of a gfx950 CU");
+    static const hipError_t attr = hipFuncSetAttribute(
+        (const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, max_lds);
+    if (attr != hipSuccess) return attr;
+    const int64_t padded = (T + KC - 1) / KC * KC;
+    const int panel = padded < kAttnPanel ? (int)padded : kAttnPanel;
+    const size_t lds = 4 * (size_t)(KC * (hd + 4) + kAttnQ * hd + kAttnQ * (panel + 4));
+    const dim3 grid((unsigned)((T + kAttnQ - 1) / kAttnQ), (unsigned)q_heads, (unsigned)batch);
+    hipLaunchKernelGGL(kern, grid, dim3(64 * kAttnQ), lds, st, q, k, v, out, T,
+                       q_heads / kv_heads, hd, q_stride, kv_stride, out_stride, window,
+                       1.0f / sqrtf((float)hd), prefix, seg_lo, seg_hi, pad, panel);
+    return hipGetLastError();
 }
 
 hipError_t launch_attention_f32(const float* q, const float* k, const float* v, float* out,
@@ -219,11 +376,15 @@ hipError_t launch_attention_f32(const float* q, const float* k, const float* v, 
                                 int64_t window, int64_t prefix, const int32_t* seg_lo,
                                 const int32_t* seg_hi, const uint64_t* pad, hipStream_t st) {
     if (window >= T) window = 0;
-    const dim3 grid((unsigned)T, (unsigned)((q_heads + 3) / 4), (unsigned)batch);
-    hipLaunchKernelGGL(attention_f32_kernel, grid, dim3(256), 0, st, q, k, v, out, T, q_heads,
-                       q_heads / kv_heads, hd, q_stride, kv_stride, out_stride, window,
-                       1.0f / sqrtf((float)hd), prefix, seg_lo, seg_hi, pad);
-    return hipGetLastError();
+#define NCM_ATTN(HS, KC)                                                                       \
+    return launch_attention_f32_t<HS, KC>(q, k, v, out, batch, T, q_heads, kv_heads, hd, q_stride, \
+                                      kv_stride, out_stride, window, prefix, seg_lo, seg_hi,   \
+                                      pad, st)
+    if (hd <= 64) NCM_ATTN(1, 128);
+    if (hd <= 128) NCM_ATTN(2, 128);
+    if (hd <= kAttnF32MaxHd) NCM_ATTN(4, 64);
+#undef NCM_ATTN
+    return hipErrorInvalidValue;
 }
 
 struct PlanF32 {
