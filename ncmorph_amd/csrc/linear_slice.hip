@@ -2,33 +2,19 @@
 // linear.hip leave most of the chip idle or multiply mostly padding (a
 // prompt of 77 tokens through a 2048-wide projection is 16 tiles for 256
 // CUs). Small output tiles fill the CUs, and the wavefronts of a workgroup
-// split K instead of the tile: wavefront w multiplies the whole tile over
-// K tiles w, w + NW, ... (64 bf16 or 32 fp32 elements each) and the NW
-// partial sums are added in wavefront order through LDS at the end, so there
-// is no second pass over memory, no workspace and no atomic.
+// split K instead of the tile (slice_partial_sums in linear_slice.h): no
+// second pass over memory, no workspace, no atomic, no barrier in the main
+// loop.
 //
 // What bounds it: the weight stream from HBM for the smallest batches, the
 // operand traffic L2 -> LDS (every column tile reads all of x, every row tile
-// all of W) for the larger ones. A wavefront's operand rows go straight to
-// its own LDS region (buffer_load ... lds, 8 rows x 128 bytes per
-// instruction: whole cache lines), NST stages deep. No other wavefront reads
-// that region, so the main loop has no barrier: each wavefront waits for its
-// oldest stage only (vmcnt), reads the stage's fragments into registers and
-// refills the stage before its MFMAs.
-//
-// Fragments: v_mfma_f32_16x16x32_bf16 (A = x rows, B = weight rows; lane l
-// supplies 16-byte chunk 4 i + l / 16 of row l % 16 for k-step i), or for
-// fp32 four v_mfma_f32_16x16x4_f32 per k-step, MFMA j taking element j of
-// each lane's chunk. D: lane l, element j holds row 4 (l / 16) + j, column
-// l % 16. LDS chunk c of row r sits at chunk c ^ ((r / 2) % 8), which gives
-// the 16 rows of a ds_read_b128 phase distinct bank groups.
+// all of W) for the larger ones, and the matrix core for fp32.
 //
 // Every output is a function of its row of x and its weight row(s) alone,
-// and of K and NW, which launch_slice takes from (M, N, K): the same sums for
-// every epilogue, so the fused results equal the unfused kernels' bit for bit.
-#include "common.h"
-#include "gemm_core.h"
+// whatever the tile: the same sums for every epilogue, so the fused results
+// equal the unfused kernels' bit for bit.
 #include "linear.h"
+#include "linear_slice.h"
 
 namespace ncm {
 
@@ -59,23 +45,8 @@ struct SliceArgs {
     int64_t seq_len, rot_cols;
 };
 
-// RB x CB blocks of 16 x 16 outputs per workgroup, NW wavefronts, NST LDS
-// stages each.
-template <bool F32, int RB, int CB, int NW, int NST>
-struct SliceShape {
-    static constexpr int ROWS = 16 * (RB + CB);
-    static constexpr int STAGE = ROWS * 128;
-    static constexpr int ND = ROWS / 8;  // load instructions per stage
-    static constexpr int RED = NW * RB * CB * 1024;
-    static constexpr int LDS = NW * NST * STAGE > RED ? NW * NST * STAGE : RED;
-    static constexpr int EPC = F32 ? 4 : 8;  // elements per 16-byte chunk
-    static_assert(LDS <= 160 * 1024, "LDS budget of a gfx950 CU");
-    static_assert(NST >= 1 && (NST - 1) * ND <= 63, "vmcnt range");
-};
-
 template <bool F32, int RB, int CB, int NW, int NST, int EPI>
 __global__ __launch_bounds__(64 * NW) void linear_slice_kernel(SliceArgs a) {
-    using S = SliceShape<F32, RB, CB, NW, NST>;
     constexpr int ESZ = F32 ? 4 : 2;
     constexpr int NB = RB * CB;
     static_assert(EPI == kPlain || CB == 2 || CB == 4, "pairs of 16-column blocks");
@@ -84,11 +55,9 @@ __global__ __launch_bounds__(64 * NW) void linear_slice_kernel(SliceArgs a) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r16 = lane & 15, grp = lane >> 4;
 
-    // The row tiles of one column tile are consecutive and on one XCD (each
-    // XCD takes a contiguous run of tiles), so W is read from HBM once.
-    const int nblk = (int)gridDim.x, bid = (int)blockIdx.x;
-    const int xcd = bid & 7, per = nblk >> 3, rem = nblk & 7;
-    const int logical = xcd * per + min(xcd, rem) + (bid >> 3);
+    // The row tiles of one column tile are consecutive and on one XCD, so W is
+    // read from HBM once.
+    const int logical = slice_logical_tile();
     const int tm = logical % a.tiles_m;
     const int tn = logical / a.tiles_m;
 
@@ -114,108 +83,9 @@ __global__ __launch_bounds__(64 * NW) void linear_slice_kernel(SliceArgs a) {
         make_rsrc((const char*)(TWO_W ? a.w2 : a.w) + n0 * K * ESZ,
                   operand_bytes(a.N, n0, K, ESZ));
 
-    // Load instruction p fills LDS rows 8 p .. 8 p + 7 (x rows, then weight
-    // rows), lane l row l / 8, chunk slot l % 8; the swizzle term depends on
-    // the parity of p only.
-    const int drow = lane >> 3;
-    const int ch0 = (lane & 7) ^ (drow >> 1), ch1 = ch0 ^ 4;
-    const uint32_t rowb = (uint32_t)(K * ESZ);
-    const uint32_t o0 = drow * rowb + ch0 * 16, o1 = drow * rowb + ch1 * 16;
-    char* region = lds + wave * (NST * S::STAGE);
-    auto dma = [&](char* stage, int64_t k0) {
-        // Chunks at or past K, and tiles past the last one, load as zero.
-        const uint32_t kb = (uint32_t)(k0 * ESZ);
-        const uint32_t v0 = k0 + ch0 * S::EPC < K ? o0 + kb : kOobOffset;
-        const uint32_t v1 = k0 + ch1 * S::EPC < K ? o1 + kb : kOobOffset;
-#pragma unroll
-        for (int p = 0; p < S::ND; ++p) {
-            const bool is_x = p < 2 * RB;
-            const int q = is_x ? p : p - 2 * RB;
-            const int cb = TWO_W ? (q >> 1) % HB : q >> 1;
-            const int row = is_x ? 8 * q : cb * BSTEP + 8 * (q & 1);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                is_x ? rsx : (TWO_W && q >= 2 * HB ? rsw2 : rsw),
-                (__attribute__((address_space(3))) void*)(stage + p * 1024), 16,
-                (p & 1 ? v1 : v0) + (uint32_t)row * rowb, 0, 0, 0);
-        }
-    };
-
-    f32x4_t acc[RB][CB];
-#pragma unroll
-    for (int i = 0; i < RB; ++i)
-#pragma unroll
-        for (int j = 0; j < CB; ++j) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-
-    constexpr int BK = 8 * S::EPC;
-    const int tiles_k = (int)((K + BK - 1) / BK);
-    const int iters = (tiles_k + NW - 1) / NW;
-#pragma unroll
-    for (int s = 0; s < NST; ++s) dma(region + s * S::STAGE, (int64_t)(wave + NW * s) * BK);
-    const uint32_t frag = (uint32_t)(r16 * 128);
-    const uint32_t c0 = (uint32_t)((grp ^ (r16 >> 1)) * 16), c1 = c0 ^ 64;
-    int st = 0;
-    for (int i = 0; i < iters; ++i) {
-        char* base = region + st * S::STAGE;
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0((NST - 1) * S::ND));
-        asm volatile("" ::: "memory");
-        u32x4_t af[2][RB], bf[2][CB];
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            const uint32_t c = ks ? c1 : c0;
-#pragma unroll
-            for (int rb = 0; rb < RB; ++rb)
-                af[ks][rb] = *(const u32x4_t*)(base + frag + rb * 2048 + c);
-#pragma unroll
-            for (int cb = 0; cb < CB; ++cb)
-                bf[ks][cb] = *(const u32x4_t*)(base + frag + (RB + cb) * 2048 + c);
-        }
-        // The stage is free once its fragments are in registers.
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        __builtin_amdgcn_sched_barrier(0);
-        dma(base, (int64_t)(wave + NW * (i + NST)) * BK);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-            for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-                for (int cb = 0; cb < CB; ++cb) {
-                    if constexpr (F32) {
-#pragma unroll
-                        for (int j = 0; j < 4; ++j)
-                            acc[rb][cb] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-                                __uint_as_float(af[ks][rb][j]), __uint_as_float(bf[ks][cb][j]),
-                                acc[rb][cb], 0, 0, 0);
-                    } else {
-                        acc[rb][cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                            __builtin_bit_cast(bf16x8_t, af[ks][rb]),
-                            __builtin_bit_cast(bf16x8_t, bf[ks][cb]), acc[rb][cb], 0, 0, 0);
-                    }
-                }
-        st = st + 1 == NST ? 0 : st + 1;
-    }
-
-    // Partial sums over the operand stages, once no load can still write
-    // there; block b of wavefront v at ((v NB + b) 64 + lane) 16 bytes.
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    f32x4_t* red = (f32x4_t*)lds;
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-        for (int cb = 0; cb < CB; ++cb) red[(wave * NB + rb * CB + cb) * 64 + lane] = acc[rb][cb];
-    __syncthreads();
-    auto sum = [&](int b) {
-        f32x4_t s = red[b * 64 + lane];
-#pragma unroll
-        for (int v = 1; v < NW; ++v) {
-            const f32x4_t p = red[(v * NB + b) * 64 + lane];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) s[j] = s[j] + p[j];
-        }
-        return s;
-    };
+    slice_partial_sums<F32, RB, CB, NW, NST, BSTEP, TWO_W>(lds, rsx, (uint32_t)(K * ESZ), rsw,
+                                                           rsw2, (uint32_t)(K * ESZ), K);
+    auto sum = [&](int b) { return slice_sum<NW, NB>(lds, b); };
     auto bias_of = [&](int64_t n) {
         if (F32) return a.bias32 ? a.bias32[n] : 0.0f;
         return a.bias ? __uint_as_float((uint32_t)a.bias[n] << 16) : 0.0f;
@@ -354,22 +224,10 @@ hipError_t launch_slice_t(SliceArgs a, hipStream_t st) {
     return hipGetLastError();
 }
 
-// Tiles RB x CB with their LDS stages. NW is 8 for all of them: the sums of
-// an output do not depend on the tile. One stage (refilled while its
-// fragments are multiplied) leaves LDS for a second workgroup on the CU up to
-// 5 blocks of rows and measured as fast as two or three from 1 x 2 up.
-constexpr int kSliceWaves = 8;
-struct Tile {
-    int rb, cb;
-};
-constexpr Tile kTiles[] = {{1, 1}, {2, 1}, {1, 2}, {2, 2}, {3, 2}, {1, 4},
-                           {4, 2}, {2, 4}, {3, 4}, {4, 4}, {5, 4}};
-constexpr int kTileCount = sizeof(kTiles) / sizeof(kTiles[0]);
-
 // Cost of a tile: rounds of the 256 CUs times the blocks of 16 operand rows
 // that a workgroup loads (at 75 GB/s a CU, over all shapes measured: 31 us for
 // 512 x 2048 x 8192 at cost 8, 18 us for 128 rows at cost 4).
-int64_t tile_cost(const Tile& s, int64_t M, int64_t N) {
+int64_t tile_cost(const SliceTile& s, int64_t M, int64_t N) {
     const int64_t tiles =
         ((M + 16 * s.rb - 1) / (16 * s.rb)) * ((N + 16 * s.cb - 1) / (16 * s.cb));
     return (tiles + 255) / 256 * (s.rb + s.cb);
@@ -378,9 +236,9 @@ int64_t tile_cost(const Tile& s, int64_t M, int64_t N) {
 // The cheapest tile (paired: one with a partner column block).
 int64_t best_tile(int64_t M, int64_t N, bool paired, int* tile) {
     int64_t best = INT64_MAX;
-    for (int t = 0; t < kTileCount; ++t) {
-        if (paired && kTiles[t].cb < 2) continue;
-        const int64_t cost = tile_cost(kTiles[t], M, N);
+    for (int t = 0; t < kSliceTileCount; ++t) {
+        if (paired && kSliceTiles[t].cb < 2) continue;
+        const int64_t cost = tile_cost(kSliceTiles[t], M, N);
         if (cost < best) {
             best = cost;
             *tile = t;
@@ -416,33 +274,6 @@ hipError_t launch_slice(int tile, const SliceArgs& a, hipStream_t st) {
         default: return hipErrorInvalidValue;
     }
 #undef NCM_SLICE
-}
-
-// fp32: the matrix core is the bound (1/16 of the bf16 rate), so a tile is
-// priced in time: rounds of the CUs times the workgroup's MFMAs (0.22 us per
-// block of 16 x 16 outputs and iteration of its eight wavefronts) plus what
-// starting, summing and storing it takes. Fitted to M = 1 .. 600 on the 135M and
-// 0.5B checkpoints' projections, within 20% where the weight stream is not the
-// bound (200 rows, 576 x 576: 4.9 us; 300 rows, 4864 x 896: 35 us).
-double f32_tile_us(const Tile& s, int64_t M, int64_t N, int64_t K) {
-    const int64_t tiles =
-        ((M + 16 * s.rb - 1) / (16 * s.rb)) * ((N + 16 * s.cb - 1) / (16 * s.cb));
-    const int64_t iters = ((K + 31) / 32 + kSliceWaves - 1) / kSliceWaves;
-    const int blocks = s.rb * s.cb;
-    return (double)((tiles + 255) / 256) * (0.22 * blocks * iters + 1.3 + 0.3 * blocks);
-}
-
-double best_tile_f32(int64_t M, int64_t N, int64_t K, bool paired, int* tile) {
-    double best = 1e300;
-    for (int t = 0; t < kTileCount; ++t) {
-        if (paired && kTiles[t].cb < 2) continue;
-        const double us = f32_tile_us(kTiles[t], M, N, K);
-        if (us < best) {
-            best = us;
-            *tile = t;
-        }
-    }
-    return best;
 }
 
 }  // namespace
@@ -506,7 +337,7 @@ bool linear_slice_f32_fits(int64_t M, int64_t N, int64_t K) {
     const int64_t big = ((M + 127) / 128) * ((N + 127) / 128);
     const double big_us = (double)((big + 255) / 256) * (2.03 * ((K + 31) / 32) + 3.5);
     int tile;
-    return best_tile_f32(M, N, K, false, &tile) < big_us;
+    return slice_best_tile_f32(M, N, K, false, &tile) < big_us;
 }
 
 hipError_t launch_linear_slice_f32(const LinearF32& l, hipStream_t st) {
@@ -518,7 +349,7 @@ hipError_t launch_linear_slice_f32(const LinearF32& l, hipStream_t st) {
     const bool rope = l.cosine != nullptr;
     if (rope && (l.N % 64 || l.rot_cols % 64 || l.seq_len <= 0)) return hipErrorInvalidValue;
     int tile = -1;
-    best_tile_f32(l.M, l.N, l.K, rope, &tile);
+    slice_best_tile_f32(l.M, l.N, l.K, rope, &tile);
     return rope ? launch_slice<kRope, true>(tile, a, st) : launch_slice<kPlain, true>(tile, a, st);
 }
 
@@ -529,7 +360,7 @@ hipError_t launch_linear_slice_swiglu_f32(const float* x, const float* gate, con
     a.x = x; a.w = gate; a.w2 = up; a.bias32 = gate_bias; a.bias2 = up_bias; a.y = y;
     a.M = M; a.K = K; a.N = N;
     int tile = -1;
-    best_tile_f32(M, 2 * N, K, true, &tile);
+    slice_best_tile_f32(M, 2 * N, K, true, &tile);
     return launch_slice<kSwiGLU, true>(tile, a, st);
 }
 

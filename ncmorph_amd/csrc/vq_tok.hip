@@ -26,6 +26,7 @@
 
 #include "gemm_core.h"
 #include "linear.h"
+#include "linear_slice.h"
 #include "status.h"
 #include "vq_tok.h"
 
@@ -81,6 +82,31 @@ __device__ __forceinline__ float gelu_exact(float x) {
 __device__ __forceinline__ float stage_value(const VtEpi& ep, float acc, int64_t n) {
     const float v = ep.bias ? acc + ep.bias[n % ep.bias_len] : acc;
     return ep.act == 1 ? gelu_exact(v) : v;
+}
+
+// One output of the stage and Phi epilogues (row m, column n of N).
+template <int EPI>
+__device__ __forceinline__ void vt_store1(const VtEpi& ep, int64_t m, int64_t n, int64_t N,
+                                          float v) {
+    if constexpr (EPI == kEpiStage) {
+        int64_t dst = m * N + n;
+        if (ep.pad_len > 0) {
+            const int64_t row = dst / ep.d;
+            dst = (row + 2 * (row / ep.pad_len) + 1) * ep.d + dst % ep.d;
+        }
+        const float o = stage_value(ep, v, n);
+        ep.y[dst] = ep.res ? ep.res[dst] + o : o;
+    } else {
+        // Virtual row m = b (L + 2) + t; t >= L straddles two sequences.
+        const int64_t b = m / (ep.seq + 2);
+        const int64_t t = m - b * (ep.seq + 2);
+        if (t >= ep.seq) return;
+        const float h = ep.hpad[(m + 1) * N + n];
+        const int64_t o = (b * ep.seq + t) * N + n;
+        const float qv = (1.0f - ep.ratio) * h + ep.ratio * (v + ep.bias[n]);
+        ep.zhat[o] = ep.first ? qv : ep.zhat[o] + qv;
+        if (ep.r) ep.r[o] = ep.r[o] - qv;
+    }
 }
 
 __device__ __forceinline__ unsigned long long shfl_xor_u64(unsigned long long v, int m) {
@@ -237,28 +263,180 @@ __attribute__((amdgpu_waves_per_eu(S::OCC, S::OCC))) void vt_gemm_kernel(
                 const int64_t m =
                     m0 + wm * S::WM + mb * 32 + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
                 if (m >= M) continue;
-                const float v = acc.v[mb][nb][i];
-                if constexpr (EPI == kEpiStage) {
-                    int64_t dst = m * N + n;
-                    if (ep.pad_len > 0) {
-                        const int64_t row = dst / ep.d;
-                        dst = (row + 2 * (row / ep.pad_len) + 1) * ep.d + dst % ep.d;
+                vt_store1<EPI>(ep, m, n, N, acc.v[mb][nb][i]);
+            }
+        }
+    }
+}
+
+// The same product and epilogues on small tiles with K split over the
+// wavefronts (linear_slice.h), for products of too few 128 x 128 tiles: Phi of
+// 24 / 96 sequences is 39 / 150 of them and took 89 / 96 us, 26 / 75 here.
+template <int RB, int CB, int NST, int EPI>
+__global__ __launch_bounds__(64 * kSliceWaves) void vt_slice_kernel(
+    const float* __restrict__ a, int64_t lda, int64_t a_rows, const float* __restrict__ w,
+    int64_t M, int64_t K, int64_t N, int tiles_m, VtEpi ep) {
+    constexpr int NB = RB * CB, NW = kSliceWaves;
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r16 = lane & 15, grp = lane >> 4;
+    const int logical = slice_logical_tile();
+    const int64_t m0 = (int64_t)(logical % tiles_m) * 16 * RB;
+    const int64_t n0 = (int64_t)(logical / tiles_m) * 16 * CB;
+    const __amdgpu_buffer_rsrc_t rsa =
+        make_rsrc((const char*)a + m0 * lda * 4, operand_bytes(a_rows, m0, lda, 4));
+    const __amdgpu_buffer_rsrc_t rsw =
+        make_rsrc((const char*)w + n0 * K * 4, operand_bytes(N, n0, K, 4));
+    // The stage and Phi epilogues' own operands, loaded before the product so
+    // that their latency hides under it: block wave + NW i of the tile, rows
+    // 4 grp + j of it.
+    constexpr int IT = EPI == kEpiDist ? 1 : (NB + NW - 1) / NW;
+    int64_t dst[IT][4];  // output element, -1: none
+    float e0[IT][4], e1[IT][4], e2[IT][4], bias[IT];
+    if constexpr (EPI == kEpiPhi) {
+        // Virtual row m = b (L + 2) + t; t >= L straddles two sequences.
+        const uint32_t period = (uint32_t)ep.seq + 2;
+        const int64_t b0 = m0 / period;
+        const uint32_t t0 = (uint32_t)(m0 - b0 * period);
+#pragma unroll
+        for (int i = 0; i < IT; ++i) {
+            const int b = wave + NW * i;
+            const int64_t n = n0 + 16 * (b % CB) + r16;
+            const bool col = b < NB && n < N;
+            bias[i] = col ? ep.bias[n] : 0.0f;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const uint32_t dr = 16 * (b / CB) + 4 * grp + j;
+                const uint32_t bq = (t0 + dr) / period, t = t0 + dr - bq * period;
+                const int64_t m = m0 + dr;
+                const bool in = col && m < M && t < (uint32_t)ep.seq;
+                dst[i][j] = in ? ((b0 + bq) * ep.seq + t) * N + n : -1;
+                e0[i][j] = in ? ep.hpad[(m + 1) * N + n] : 0.0f;
+                e1[i][j] = in && !ep.first ? ep.zhat[dst[i][j]] : 0.0f;
+                e2[i][j] = in && ep.r ? ep.r[dst[i][j]] : 0.0f;
+            }
+        }
+    } else if constexpr (EPI == kEpiStage) {
+        // pad_len > 0: flat row R = (m N + n) / D of [rows, D] at padded row
+        // R + 2 (R / pad_len) + 1; N is s D.
+        const uint32_t d = (uint32_t)ep.d, sd = (uint32_t)N / d;
+        const int64_t R0 = m0 * sd;
+        const uint32_t pl = ep.pad_len > 0 ? (uint32_t)ep.pad_len : 1u;
+        const int64_t q0 = R0 / pl;
+        const uint32_t u0 = (uint32_t)(R0 - q0 * pl);
+#pragma unroll
+        for (int i = 0; i < IT; ++i) {
+            const int b = wave + NW * i;
+            const int64_t n = n0 + 16 * (b % CB) + r16;
+            const bool col = b < NB && n < N;
+            bias[i] = col && ep.bias ? ep.bias[(uint32_t)n % (uint32_t)ep.bias_len] : 0.0f;
+            const uint32_t nj = (uint32_t)n / d;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const uint32_t dr = 16 * (b / CB) + 4 * grp + j;
+                const int64_t m = m0 + dr;
+                int64_t o = m * N + n;
+                if (ep.pad_len > 0) o += (2 * (q0 + (u0 + dr * sd + nj) / pl) + 1) * (int64_t)d;
+                dst[i][j] = col && m < M ? o : -1;
+                e0[i][j] = dst[i][j] >= 0 && ep.res ? ep.res[o] : 0.0f;
+            }
+        }
+    }
+    slice_partial_sums<true, RB, CB, NW, NST, 16, false>(lds, rsa, (uint32_t)(lda * 4), rsw, rsw,
+                                                         (uint32_t)(K * 4), K);
+    if constexpr (EPI == kEpiDist) {
+        // Wavefront rb: the minimum key of 16 rows over the tile's columns. A
+        // lane holds rows 4 grp + j of column r16 of each block; two halving
+        // exchanges over the 16 lanes leave one row a lane, two more its
+        // minimum over the four lanes that hold it.
+        for (int rb = wave; rb < RB; rb += NW) {
+            unsigned long long k4[4] = {~0ull, ~0ull, ~0ull, ~0ull};
+#pragma unroll
+            for (int cb = 0; cb < CB; ++cb) {
+                const int64_t n = n0 + 16 * cb + r16;
+                const f32x4_t v = slice_sum<NW, NB>(lds, rb * CB + cb);
+                if (n < N) {
+                    const float c = ep.csq[n];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const unsigned long long k = dist_key(c - 2.0f * v[j], n);
+                        k4[j] = k < k4[j] ? k : k4[j];
                     }
-                    const float o = stage_value(ep, v, n);
-                    ep.y[dst] = ep.res ? ep.res[dst] + o : o;
+                }
+            }
+            auto meet = [&](unsigned long long keep, unsigned long long send, int x) {
+                const unsigned long long recv = shfl_xor_u64(send, x);
+                return recv < keep ? recv : keep;
+            };
+            const bool up8 = (lane & 8) != 0, up4 = (lane & 4) != 0;
+            const unsigned long long p0 = meet(up8 ? k4[2] : k4[0], up8 ? k4[0] : k4[2], 8);
+            const unsigned long long p1 = meet(up8 ? k4[3] : k4[1], up8 ? k4[1] : k4[3], 8);
+            unsigned long long best = meet(up4 ? p1 : p0, up4 ? p0 : p1, 4);
+            best = meet(best, best, 2);
+            best = meet(best, best, 1);
+            const int64_t m = m0 + 16 * rb + 4 * grp + (up8 ? 2 : 0) + (up4 ? 1 : 0);
+            if ((lane & 3) == 0 && m < M && best != ~0ull) atomicMin(ep.keys + m, best);
+        }
+        return;
+    } else {
+#pragma unroll
+        for (int i = 0; i < IT; ++i) {
+            const int b = wave + NW * i;
+            if (b >= NB) break;
+            const f32x4_t v = slice_sum<NW, NB>(lds, b);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int64_t o = dst[i][j];
+                if (o < 0) continue;
+                if constexpr (EPI == kEpiPhi) {
+                    const float q = (1.0f - ep.ratio) * e0[i][j] + ep.ratio * (v[j] + bias[i]);
+                    ep.zhat[o] = ep.first ? q : e1[i][j] + q;
+                    if (ep.r) ep.r[o] = e2[i][j] - q;
                 } else {
-                    const int64_t b = m / (ep.seq + 2);
-                    const int64_t t = m - b * (ep.seq + 2);
-                    if (t >= ep.seq) continue;
-                    const float h = ep.hpad[(m + 1) * N + n];
-                    const int64_t o = (b * ep.seq + t) * N + n;
-                    const float qv = (1.0f - ep.ratio) * h + ep.ratio * (v + ep.bias[n]);
-                    ep.zhat[o] = ep.first ? qv : ep.zhat[o] + qv;
-                    if (ep.r) ep.r[o] = ep.r[o] - qv;
+                    const float x = ep.bias ? v[j] + bias[i] : v[j];
+                    const float y = ep.act == 1 ? gelu_exact(x) : x;
+                    ep.y[o] = ep.res ? e0[i][j] + y : y;
                 }
             }
         }
     }
+}
+
+template <int RB, int CB, int NST, int EPI>
+hipError_t launch_vt_slice_t(const float* a, int64_t lda, int64_t a_rows, const float* w,
+                             int64_t M, int64_t K, int64_t N, const VtEpi& ep, hipStream_t st) {
+    using S = SliceShape<true, RB, CB, kSliceWaves, NST>;
+    auto kern = vt_slice_kernel<RB, CB, NST, EPI>;
+    static const hipError_t attr = hipFuncSetAttribute(
+        (const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, S::LDS);
+    if (attr != hipSuccess) return attr;
+    const int tiles_m = (int)((M + 16 * RB - 1) / (16 * RB));
+    const int64_t blocks = tiles_m * ((N + 16 * CB - 1) / (16 * CB));
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(64 * kSliceWaves), S::LDS, st, a, lda,
+                       a_rows, w, M, K, N, tiles_m, ep);
+    return hipGetLastError();
+}
+
+template <int EPI>
+hipError_t launch_vt_slice(int tile, const float* a, int64_t lda, int64_t a_rows, const float* w,
+                           int64_t M, int64_t K, int64_t N, const VtEpi& ep, hipStream_t st) {
+#define VT_SLICE(RB, CB, NST) \
+    return launch_vt_slice_t<RB, CB, NST, EPI>(a, lda, a_rows, w, M, K, N, ep, st)
+    switch (tile) {
+        case 0: VT_SLICE(1, 1, 2);
+        case 1: VT_SLICE(2, 1, 1);
+        case 2: VT_SLICE(1, 2, 1);
+        case 3: VT_SLICE(2, 2, 1);
+        case 4: VT_SLICE(3, 2, 1);
+        case 5: VT_SLICE(1, 4, 1);
+        case 6: VT_SLICE(4, 2, 1);
+        case 7: VT_SLICE(2, 4, 1);
+        case 8: VT_SLICE(3, 4, 1);
+        case 9: VT_SLICE(4, 4, 1);
+        default: VT_SLICE(5, 4, 1);
+    }
+#undef VT_SLICE
 }
 
 template <int EPI>
@@ -277,6 +455,13 @@ hipError_t launch_vt_gemm(const float* a, int64_t lda, int64_t a_rows, const flo
     if (M <= 0 || N <= 0) return hipSuccess;
     const int tiles_m = (int)((M + S::BM - 1) / S::BM);
     const int tiles_n = (int)((N + S::BN - 1) / S::BN);
+    // A round of 128 x 128 tiles: 2.6 us per 32 elements of K (96 us for up to
+    // 256 tiles at K = 1152).
+    const double big_us =
+        (double)(((int64_t)tiles_m * tiles_n + 255) / 256) * (2.6 * ((K + 31) / 32) + 4.0);
+    int tile = -1;
+    if (K > 0 && slice_best_tile_f32(M, N, K, false, &tile) < big_us)
+        return launch_vt_slice<EPI>(tile, a, lda, a_rows, w, M, K, N, ep, st);
     const int group_m = tiles_m < 4 ? tiles_m : 4;
     hipLaunchKernelGGL(kern, dim3(tiles_m * tiles_n), dim3(S::NT), S::LDS_BYTES, st, a, lda,
                        a_rows, w, M, K, N, tiles_n, group_m, ep);
