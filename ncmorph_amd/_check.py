@@ -9,8 +9,6 @@ layout, so that the checks also run without a GPU.
 """
 from __future__ import annotations
 
-import ctypes as C
-
 from ._lib import NCM_E_ARG, NCM_E_NULL, NCM_E_SHAPE, NcmError
 
 # bf16 operands travel as 16-bit patterns: torch.bfloat16, or an int16 /
@@ -21,8 +19,14 @@ I32 = ("int32",)
 U64 = ("int64", "uint64")
 
 
+_NAMES = {}  # a dtype object's name, as met
+
+
 def _dtype(t) -> str:
-    return str(t.dtype).replace("torch.", "")
+    name = _NAMES.get(t.dtype)
+    if name is None:
+        name = _NAMES[t.dtype] = str(t.dtype).replace("torch.", "")
+    return name
 
 
 def _common(t, name, where, dtypes):
@@ -50,7 +54,7 @@ class Args:
         self.seen = []
 
     def dev(self, t, name, dtypes, shape=None, optional=False):
-        """Pointer of a contiguous tensor of one of `dtypes` and exactly
+        """Address of a contiguous tensor of one of `dtypes` and exactly
         `shape` (None: any shape); None for an optional None."""
         W = self.where
         if t is None:
@@ -58,16 +62,16 @@ class Args:
                 return None
             raise NcmError(NCM_E_NULL, W, f"{name} is required")
         _common(t, name, W, dtypes)
-        if shape is not None and tuple(t.shape) != tuple(int(s) for s in shape):
+        if shape is not None and tuple(t.shape) != tuple(shape):
             raise NcmError(NCM_E_SHAPE, W,
                            f"{name} has shape {tuple(t.shape)}, expected {tuple(shape)}")
         if not t.is_contiguous():
             raise NcmError(NCM_E_ARG, W, f"{name} must be contiguous")
         self.seen.append((t, name))
-        return C.c_void_p(t.data_ptr())
+        return t.data_ptr()
 
     def rows(self, t, name, dtypes, n_rows, min_cols):
-        """(pointer, row stride) of a 2-D tensor with contiguous rows (a
+        """(address, row stride) of a 2-D tensor with contiguous rows (a
         column slice of a wider buffer is allowed): exactly n_rows rows of
         at least min_cols elements."""
         W = self.where
@@ -80,7 +84,7 @@ class Args:
         if t.stride(1) != 1 or (n_rows > 1 and t.stride(0) < min_cols):
             raise NcmError(NCM_E_ARG, W, f"{name} must have contiguous, non-overlapping rows")
         self.seen.append((t, name))
-        return C.c_void_p(t.data_ptr()), t.stride(0)
+        return t.data_ptr(), t.stride(0)
 
     def done(self):
         device = self.seen[0][0].device if self.seen else None
@@ -94,4 +98,4 @@ def dims(t, name, where, ndim):
         raise NcmError(NCM_E_NULL, where, f"{name} is required")
     if not hasattr(t, "shape") or len(t.shape) != ndim:
         raise NcmError(NCM_E_SHAPE, where, f"{name} must have {ndim} dimensions")
-    return tuple(int(s) for s in t.shape)
+    return tuple(map(int, t.shape))

@@ -7,6 +7,22 @@ import threading
 from ._lib import check, lib
 
 
+_raw_stream = None
+
+
+def _current_stream(device: int) -> int:
+    """Handle of torch's current stream on `device`. torch's own raw lookup
+    where it has one: current_stream() builds a Stream object each time, a
+    good part of a short call's host time."""
+    global _raw_stream
+    if _raw_stream is None:
+        import torch
+
+        _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (
+            lambda d: torch.cuda.current_stream(d).cuda_stream)
+    return _raw_stream(device)
+
+
 class Context:
     """Owns an ncm_ctx_t. Each call runs on torch's current stream of the
     context's device, so library kernels order with torch's own work."""
@@ -21,11 +37,10 @@ class Context:
     def bind_stream(self, stream=None) -> None:
         """Route library work to `stream` (a torch.cuda.Stream) or to torch's
         current stream on this device."""
-        import torch
-
-        if stream is None:
-            stream = torch.cuda.current_stream(self.device)
-        h = stream.cuda_stream
+        if stream is not None:
+            h = stream.cuda_stream
+        else:
+            h = _current_stream(self.device)
         if h != self._bound:
             check(lib().ncm_set_stream(self.handle, C.c_void_p(h)), "ncm_set_stream")
             self._bound = h
