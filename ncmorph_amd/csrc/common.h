@@ -50,23 +50,69 @@ __device__ __forceinline__ float flush_subnormal(float v) {
     return (b & 0x7F800000u) == 0 ? __uint_as_float(b & 0x80000000u) : v;
 }
 
+// v + b with subnormal sums flushed, for 16 values at once: one branch that
+// is hardly ever taken instead of four operations a value (the test: with the
+// sign shifted out and 1 taken off, exactly the subnormals lie below 2^24 - 1).
+__device__ __forceinline__ void add_flush16(f32x16_t& v, float b) {
+    uint32_t mn = 0xFFFFFFFFu;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        v[i] = v[i] + b;
+        mn = min(mn, (__float_as_uint(v[i]) << 1) - 1u);
+    }
+    if (__builtin_expect(__ballot(mn < 0x00FFFFFFu) != 0ull, 0)) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) v[i] = flush_subnormal(v[i]);
+    }
+}
+
+// g / (1 + exp(-g)), to be rounded to bf16: exp(-g) as exp2 of -g times the
+// upper 16 bits of log2 e (exact in fp32 for a bf16 g, which has 8 bits), corrected to first order for the rest, and v_rcp_f32 for the
+// division; about 2 fp32 ulps in all, at a third of expf and the IEEE
+// division's instructions. Over all 65,280 finite g the bf16 result is that of
+// the exact quotient but for at most two within 2 ulps of a rounding boundary.
+// Past |g| = 150 the exponential has saturated (the clamp keeps its correction
+// from being infinity times zero).
+// EXACT_G: g is a bf16 value; else any fp32 value, whose rounding in the
+// product with the upper bits is put back too (the same result for a bf16 g).
+template <bool EXACT_G = true>
+__device__ __forceinline__ float silu_near(float g) {
+    constexpr float kHi = 1.44268798828125f;  // 47274 / 32768
+    constexpr float kLoLn2 = 4.8884952e-06f;  // (log2 e - kHi) ln 2
+    const float n = -__builtin_amdgcn_fmed3f(g, -150.0f, 150.0f);
+    const float t = n * kHi;
+    const float e = __builtin_amdgcn_exp2f(t);
+    float c = n * kLoLn2;
+    if (!EXACT_G) c = __builtin_fmaf(__builtin_fmaf(n, kHi, -t), 0.6931471806f, c);
+    // A quarter of both sides: the reciprocal of the largest finite sum is then
+    // still a normal number (v_rcp_f32 has no subnormal results).
+    return (0.25f * g) * __builtin_amdgcn_rcpf(__builtin_fmaf(__builtin_fmaf(e, c, e), 0.25f, 0.25f));
+}
+
 // round(silu_bf16(gate) * up) of two elements from their accumulators
 // (packages/kernels/root.zig:265-270, src/decoder.zig:210-211): the gate and
-// up projections' bits (bf16(flush(acc + bias))), a = rb(g / (1 + expf(-g)))
+// up projections' bits (bf16(flush(acc + bias))), a = rb(silu_near(g))
 // with rb(v) = v rounded to a bf16 value, then round(a * up); the roundings
 // two values per v_cvt_pk_bf16_f32, bit for bit the same as bf16_bits_rne
 // (the unfused SiLU x up kernel's arithmetic).
-__device__ __forceinline__ void swiglu_bits2(float ga0, float ua0, float ga1, float ua1,
-                                             float bg, float bu, uint32_t& o0, uint32_t& o1) {
+// swiglu_bits2_flushed: the sums with their bias and flush already applied.
+__device__ __forceinline__ uint32_t swiglu_bits2_flushed(float ga0, float ua0, float ga1,
+                                                         float ua1) {
     // Intermediate roundings without the NaN rule: a NaN stays a NaN through
     // the products and the quotient, and the final rounding maps it to 0x7FC0.
-    const uint32_t p0 = bf16x2_rne(flush_subnormal(ga0 + bg), flush_subnormal(ua0 + bu));
-    const uint32_t p1 = bf16x2_rne(flush_subnormal(ga1 + bg), flush_subnormal(ua1 + bu));
+    const uint32_t p0 = bf16x2_rne(ga0, ua0);
+    const uint32_t p1 = bf16x2_rne(ga1, ua1);
     const float g0 = __uint_as_float(p0 << 16), u0 = __uint_as_float(p0 & 0xFFFF0000u);
     const float g1 = __uint_as_float(p1 << 16), u1 = __uint_as_float(p1 & 0xFFFF0000u);
-    const uint32_t a = bf16x2_rne(g0 / (1.0f + expf(-g0)), g1 / (1.0f + expf(-g1)));
-    const uint32_t r = bf16x2_bits_rne(__uint_as_float(a << 16) * u0,
-                                       __uint_as_float(a & 0xFFFF0000u) * u1);
+    const uint32_t a = bf16x2_rne(silu_near(g0), silu_near(g1));
+    return bf16x2_bits_rne(__uint_as_float(a << 16) * u0,
+                           __uint_as_float(a & 0xFFFF0000u) * u1);
+}
+__device__ __forceinline__ void swiglu_bits2(float ga0, float ua0, float ga1, float ua1,
+                                             float bg, float bu, uint32_t& o0, uint32_t& o1) {
+    const uint32_t r =
+        swiglu_bits2_flushed(flush_subnormal(ga0 + bg), flush_subnormal(ua0 + bu),
+                             flush_subnormal(ga1 + bg), flush_subnormal(ua1 + bu));
     o0 = r & 0xFFFFu;
     o1 = r >> 16;
 }

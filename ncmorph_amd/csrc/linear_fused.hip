@@ -67,46 +67,53 @@ __attribute__((amdgpu_waves_per_eu(S::OCC, S::OCC))) void linear_pair_kernel(
     const int c = lane & 31;
     const int64_t ld = EPI == kEpiSwiGLU ? N / 2 : N;
 
+    // Per group of 4 rows: a quad transpose leaves each lane with 4
+    // consecutive columns of one row, so stores are 8 bytes and each RoPE
+    // table half is one 16-byte load. Rows past M (a partial last row tile)
+    // are computed on table row 0 and not stored.
+    const int q = lane & 3;
+    const int hrow = 4 * (lane >> 5) + q;
+    const int c4 = c & ~3;
+    // First column of pair p's first tile; N % 64 == 0: the pair is wholly in
+    // or out (wave-uniform).
+    auto col_of = [&](int p) { return n0 + wn * S::WN + 64 * p; };
+    // bf16(flush(acc + bias)) is what the projection writes.
 #pragma unroll
     for (int p = 0; p < S::NB / 2; ++p) {
-        const int64_t col_a = n0 + wn * S::WN + 64 * p + c;  // first tile's column
-        // N % 64 == 0: the pair is wholly in or out (wave-uniform).
-        const bool in_range = col_a < N;
+        const int64_t col = col_of(p) + c;
         float ba = 0.0f, bb = 0.0f;
-        if (HAS_BIAS && in_range) {
-            ba = __uint_as_float((uint32_t)bias[col_a] << 16);
-            bb = __uint_as_float((uint32_t)bias[col_a + 32] << 16);
+        if (HAS_BIAS && col < N) {
+            ba = __uint_as_float((uint32_t)bias[col] << 16);
+            bb = __uint_as_float((uint32_t)bias[col + 32] << 16);
         }
-        const bool rotate = EPI == kEpiRope && col_a < pa.rot_cols;
 #pragma unroll
         for (int mb = 0; mb < S::MB; ++mb) {
-            if (!in_range) break;
-            // Per group of 4 rows: the projection's bits, a quad transpose
-            // (each lane then holds 4 consecutive columns of one row, so
-            // stores are 8 bytes and each RoPE table half is one 16-byte
-            // load), then the fused op. Rows past M (a partial last row
-            // tile) are computed on table row 0 and not stored.
-            const int q = lane & 3;
-            const int hrow = 4 * (lane >> 5) + q;
-            const int c4 = c & ~3;
-            const int64_t ca = EPI == kEpiSwiGLU ? (n0 + wn * S::WN) / 2 + 32 * p + c4
-                                                 : col_a - c + c4;
+            add_flush16(acc.v[mb][2 * p], ba);
+            add_flush16(acc.v[mb][2 * p + 1], bb);
+        }
+    }
+
+    if constexpr (EPI == kEpiSwiGLU) {
+        // Elementwise first (gate and up of a column sit in the same lane and
+        // element), then one transpose of the results.
 #pragma unroll
-            for (int blk = 0; blk < 4; ++blk) {
-                const int64_t m = m0 + wm * S::WM + mb * 32 + 8 * blk + hrow;
-                if (EPI == kEpiSwiGLU) {
-                    // Elementwise first (gate and up of a column sit in the
-                    // same lane and element), then one transpose of the
-                    // results.
+        for (int p = 0; p < S::NB / 2; ++p) {
+            if (col_of(p) >= N) break;
+            const int64_t ca = (n0 + wn * S::WN) / 2 + 32 * p + c4;
+#pragma unroll
+            for (int mb = 0; mb < S::MB; ++mb)
+#pragma unroll
+                for (int blk = 0; blk < 4; ++blk) {
+                    const int64_t m = m0 + wm * S::WM + mb * 32 + 8 * blk + hrow;
                     float r[4];
 #pragma unroll
                     for (int j = 0; j < 4; j += 2) {
-                        uint32_t o0, o1;
-                        swiglu_bits2(acc.v[mb][2 * p][4 * blk + j], acc.v[mb][2 * p + 1][4 * blk + j],
-                                     acc.v[mb][2 * p][4 * blk + j + 1],
-                                     acc.v[mb][2 * p + 1][4 * blk + j + 1], ba, bb, o0, o1);
-                        r[j] = __uint_as_float(o0);
-                        r[j + 1] = __uint_as_float(o1);
+                        const int i = 4 * blk + j;
+                        const uint32_t o = swiglu_bits2_flushed(
+                            acc.v[mb][2 * p][i], acc.v[mb][2 * p + 1][i],
+                            acc.v[mb][2 * p][i + 1], acc.v[mb][2 * p + 1][i + 1]);
+                        r[j] = __uint_as_float(o & 0xFFFFu);
+                        r[j + 1] = __uint_as_float(o >> 16);
                     }
                     quad_transpose4(r, q);
                     if (m < M) {
@@ -115,55 +122,66 @@ __attribute__((amdgpu_waves_per_eu(S::OCC, S::OCC))) void linear_pair_kernel(
                         o[1] = __float_as_uint(r[2]) | (__float_as_uint(r[3]) << 16);
                         __builtin_nontemporal_store(o, (u32x2_t*)(y + m * ld + ca));
                     }
-                    continue;
                 }
-                // The two tiles' projection bits, bf16(flush(acc + bias)), one
-                // v_cvt_pk_bf16_f32 per pair.
-                float va[4], vb[4];
+        }
+        return;
+    }
+
+    // RoPE. The table row of a group of rows is loaded and rounded once for
+    // all heads of the wavefront; its number is a 32-bit remainder from the
+    // tile's first row's.
+    const uint32_t seq = (uint32_t)pa.seq_len;
+    const uint32_t t0 = (uint32_t)(m0 % pa.seq_len);
+    const bool any_rot = col_of(0) < pa.rot_cols;
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const uint32_t pr =
-                        bf16x2_bits_rne(flush_subnormal(acc.v[mb][2 * p][4 * blk + j] + ba),
-                                        flush_subnormal(acc.v[mb][2 * p + 1][4 * blk + j] + bb));
-                    va[j] = __uint_as_float(pr & 0xFFFFu);
-                    vb[j] = __uint_as_float(pr >> 16);
-                }
-                quad_transpose4(va, q);
-                quad_transpose4(vb, q);
-                // Two columns per register from here on.
-                uint32_t ra[2], rbits[2];
+    for (int mb = 0; mb < S::MB; ++mb)
+#pragma unroll
+        for (int blk = 0; blk < 4; ++blk) {
+            const uint32_t dr = wm * S::WM + mb * 32 + 8 * blk + hrow;
+            const int64_t m = m0 + dr;
+            uint32_t tc[2], ts[2], tc2[2], ts2[2];
+            if (any_rot) {
+                const uint32_t t = m < M ? (t0 + dr) % seq : 0u;
+                const float* ct = pa.cosine + (int64_t)t * 64 + c4;
+                const float* st = pa.sine + (int64_t)t * 64 + c4;
+                const f32x4_t cf = *(const f32x4_t*)ct, cs = *(const f32x4_t*)(ct + 32);
+                const f32x4_t sf = *(const f32x4_t*)st, ss = *(const f32x4_t*)(st + 32);
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
-                    ra[h] = __float_as_uint(va[2 * h]) | (__float_as_uint(va[2 * h + 1]) << 16);
-                    rbits[h] = __float_as_uint(vb[2 * h]) | (__float_as_uint(vb[2 * h + 1]) << 16);
+                    tc[h] = bf16x2_rne(cf[2 * h], cf[2 * h + 1]);
+                    ts[h] = bf16x2_rne(sf[2 * h], sf[2 * h + 1]);
+                    tc2[h] = bf16x2_rne(cs[2 * h], cs[2 * h + 1]);
+                    ts2[h] = bf16x2_rne(ss[2 * h], ss[2 * h + 1]);
                 }
-                if (rotate) {
-                    const int64_t t = (m < M ? m : 0) % pa.seq_len;
-                    const f32x4_t cf = *(const f32x4_t*)(pa.cosine + t * 64 + c4);
-                    const f32x4_t cs = *(const f32x4_t*)(pa.cosine + t * 64 + 32 + c4);
-                    const f32x4_t sf = *(const f32x4_t*)(pa.sine + t * 64 + c4);
-                    const f32x4_t ss = *(const f32x4_t*)(pa.sine + t * 64 + 32 + c4);
+            }
 #pragma unroll
-                    for (int h = 0; h < 2; ++h)
-                        rope_bits2(ra[h], rbits[h], bf16x2_rne(cf[2 * h], cf[2 * h + 1]),
-                                   bf16x2_rne(sf[2 * h], sf[2 * h + 1]),
-                                   bf16x2_rne(cs[2 * h], cs[2 * h + 1]),
-                                   bf16x2_rne(ss[2 * h], ss[2 * h + 1]));
+            for (int p = 0; p < S::NB / 2; ++p) {
+                if (col_of(p) >= N) break;
+                // The two tiles' bits of a row in one register through the
+                // transpose, then two columns per register.
+                float v[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    v[j] = __uint_as_float(bf16x2_bits_rne(acc.v[mb][2 * p][4 * blk + j],
+                                                           acc.v[mb][2 * p + 1][4 * blk + j]));
+                quad_transpose4(v, q);
+                u32x2_t ra, rb;
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const uint32_t e = __float_as_uint(v[2 * h]), o = __float_as_uint(v[2 * h + 1]);
+                    uint32_t lo = __builtin_amdgcn_perm(o, e, 0x05040100u);
+                    uint32_t hi = __builtin_amdgcn_perm(o, e, 0x07060302u);
+                    if (col_of(p) < pa.rot_cols) rope_bits2(lo, hi, tc[h], ts[h], tc2[h], ts2[h]);
+                    ra[h] = lo;
+                    rb[h] = hi;
                 }
                 if (m < M) {
-                    u32x2_t o;
-                    o[0] = ra[0];
-                    o[1] = ra[1];
-                    __builtin_nontemporal_store(o, (u32x2_t*)(y + m * ld + ca));
-                    if (EPI == kEpiRope) {
-                        o[0] = rbits[0];
-                        o[1] = rbits[1];
-                        __builtin_nontemporal_store(o, (u32x2_t*)(y + m * ld + ca + 32));
-                    }
+                    uint16_t* dst = y + m * ld + col_of(p) + c4;
+                    __builtin_nontemporal_store(ra, (u32x2_t*)dst);
+                    __builtin_nontemporal_store(rb, (u32x2_t*)(dst + 32));
                 }
             }
         }
-    }
 }
 
 template <class S, int EPI, bool HAS_BIAS>
