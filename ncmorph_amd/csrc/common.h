@@ -272,11 +272,12 @@ __device__ __forceinline__ double wave_sum_xor_d(double v) {
 }
 
 // Remap a linear workgroup id so that consecutive logical tiles land on the
-// same XCD (workgroups are dispatched round-robin over the 8 XCDs).
+// same XCD (workgroups are dispatched round-robin over the 8 XCDs): XCD x takes
+// the run of nblk / 8 ids, one more for the first nblk % 8 of them, that
+// follows XCD x - 1's.
 __device__ __forceinline__ int xcd_remap(int bid, int nblk) {
-    constexpr int kXcd = 8;
-    if (nblk % kXcd != 0) return bid;
-    return (bid % kXcd) * (nblk / kXcd) + bid / kXcd;
+    const int x = bid & 7, per = nblk >> 3, rem = nblk & 7;
+    return x * per + min(x, rem) + (bid >> 3);
 }
 
 }  // namespace ncm

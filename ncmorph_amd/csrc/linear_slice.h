@@ -36,13 +36,6 @@ struct SliceShape {
     static_assert(NST >= 1 && (NST - 1) * ND <= 63, "vmcnt range");
 };
 
-// Logical tile of this workgroup: each XCD takes a contiguous run of tiles.
-__device__ __forceinline__ int slice_logical_tile() {
-    const int nblk = (int)gridDim.x, bid = (int)blockIdx.x;
-    const int xcd = bid & 7, per = nblk >> 3, rem = nblk & 7;
-    return xcd * per + min(xcd, rem) + (bid >> 3);
-}
-
 // The tile's partial sums into LDS: block b of wavefront v at ((v NB + b) 64 +
 // lane) 16 bytes; the barrier that ends it makes them visible. rsx: the 16 RB
 // rows of A, xstride bytes apart; rsw: 16 CB rows of B, wstride bytes apart,
@@ -188,15 +181,16 @@ constexpr int kSliceTileCount = sizeof(kSliceTiles) / sizeof(kSliceTiles[0]);
 // fp32: the matrix core is the bound (1/16 of the bf16 rate), so a tile is
 // priced in time: rounds of the CUs times the workgroup's MFMAs (0.22 us per
 // block of 16 x 16 outputs and iteration of its eight wavefronts) plus what
-// starting, summing and storing it takes. Fitted to M = 1 .. 600 on the 135M and
-// 0.5B checkpoints' projections, within 20% where the weight stream is not the
-// bound (200 rows, 576 x 576: 4.9 us; 300 rows, 4864 x 896: 35 us).
+// starting, summing and storing it takes, plus the launch. Fitted to M = 1 ..
+// 600 on the 135M and 0.5B checkpoints' projections, within 20% where the
+// weight stream is not the bound (200 rows, 576 x 576: 4.9 us + launch; 300 rows,
+// 4864 x 896: 35 us).
 inline double slice_f32_tile_us(const SliceTile& s, int64_t M, int64_t N, int64_t K) {
     const int64_t tiles =
         ((M + 16 * s.rb - 1) / (16 * s.rb)) * ((N + 16 * s.cb - 1) / (16 * s.cb));
     const int64_t iters = ((K + 31) / 32 + kSliceWaves - 1) / kSliceWaves;
     const int blocks = s.rb * s.cb;
-    return (double)((tiles + 255) / 256) * (0.22 * blocks * iters + 1.3 + 0.3 * blocks);
+    return 3.0 + (double)((tiles + 255) / 256) * (0.22 * blocks * iters + 1.3 + 0.3 * blocks);
 }
 
 inline double slice_best_tile_f32(int64_t M, int64_t N, int64_t K, bool paired, int* tile) {

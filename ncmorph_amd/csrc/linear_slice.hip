@@ -57,7 +57,7 @@ __global__ __launch_bounds__(64 * NW) void linear_slice_kernel(SliceArgs a) {
 
     // The row tiles of one column tile are consecutive and on one XCD, so W is
     // read from HBM once.
-    const int logical = slice_logical_tile();
+    const int logical = xcd_remap((int)blockIdx.x, (int)gridDim.x);
     const int tm = logical % a.tiles_m;
     const int tn = logical / a.tiles_m;
 
@@ -335,7 +335,7 @@ hipError_t launch_linear_slice_rope64(const uint16_t* x, const uint16_t* w, cons
 bool linear_slice_f32_fits(int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || N <= 0 || K <= 0 || K > (int64_t)1 << 20) return false;
     const int64_t big = ((M + 127) / 128) * ((N + 127) / 128);
-    const double big_us = (double)((big + 255) / 256) * (2.03 * ((K + 31) / 32) + 3.5);
+    const double big_us = (double)((big + 255) / 256) * (2.03 * ((K + 31) / 32) + 3.5) + 3.0;
     int tile;
     return slice_best_tile_f32(M, N, K, false, &tile) < big_us;
 }

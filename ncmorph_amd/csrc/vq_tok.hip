@@ -281,7 +281,7 @@ __global__ __launch_bounds__(64 * kSliceWaves) void vt_slice_kernel(
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r16 = lane & 15, grp = lane >> 4;
-    const int logical = slice_logical_tile();
+    const int logical = xcd_remap((int)blockIdx.x, (int)gridDim.x);
     const int64_t m0 = (int64_t)(logical % tiles_m) * 16 * RB;
     const int64_t n0 = (int64_t)(logical / tiles_m) * 16 * CB;
     const __amdgpu_buffer_rsrc_t rsa =
@@ -458,7 +458,7 @@ hipError_t launch_vt_gemm(const float* a, int64_t lda, int64_t a_rows, const flo
     // A round of 128 x 128 tiles: 2.6 us per 32 elements of K (96 us for up to
     // 256 tiles at K = 1152).
     const double big_us =
-        (double)(((int64_t)tiles_m * tiles_n + 255) / 256) * (2.6 * ((K + 31) / 32) + 4.0);
+        (double)(((int64_t)tiles_m * tiles_n + 255) / 256) * (2.6 * ((K + 31) / 32) + 4.0) + 3.0;
     int tile = -1;
     if (K > 0 && slice_best_tile_f32(M, N, K, false, &tile) < big_us)
         return launch_vt_slice<EPI>(tile, a, lda, a_rows, w, M, K, N, ep, st);
