@@ -145,7 +145,8 @@ struct SegArgs {
 template <int HD>
 constexpr bool attn_dyn_lds() { return HD == 128; }
 
-template <int HD, int OUT_MODE, int MASK, int NWV, bool POW2 = (HD == 64)>
+template <int HD, int OUT_MODE, int MASK, int NWV, bool PAIR = (MASK == 0),
+          bool POW2 = (HD == 64)>
 __global__ __launch_bounds__(64 * NWV)
 __attribute__((amdgpu_waves_per_eu(2, 4))) void attention_bf16_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
@@ -236,15 +237,16 @@ __attribute__((amdgpu_waves_per_eu(2, 4))) void attention_bf16_kernel(
         return a;
     };
 
-    // Causal balance: workgroup x takes query block nqb - 1 - x (the most
+    // Causal balance (PAIR): workgroup x takes query block nqb - 1 - x (the most
     // keys) and then block x (the fewest), so every workgroup walks about
     // the same number of key blocks (the middle block of an odd count is
-    // taken once). Level mask: one query block per workgroup, the last
-    // (longest level) blocks first.
+    // taken once). Without PAIR (few enough workgroups to be resident
+    // together, or the level mask): one query block per workgroup, the last
+    // (longest) blocks first.
     const int nqb = (int)((T + kBq - 1) / kBq);
     for (int part = 0; part < 2; ++part) {
     const int qbi = part == 0 ? nqb - 1 - xb : xb;
-    if (part == 1 && (MASK == 1 || qbi == nqb - 1 - xb)) break;
+    if (part == 1 && (!PAIR || qbi == nqb - 1 - xb)) break;
     const int64_t q0 = (int64_t)qbi * kBq;
     const int64_t qw0 = q0 + 32 * wave;
     const int64_t qq = qw0 + c;  // the query of this lane's score column
@@ -550,6 +552,181 @@ __attribute__((amdgpu_waves_per_eu(2, 4))) void attention_bf16_kernel(
     }  // part
 }
 
+namespace {
+
+// Causal attention of short sequences (up to 32 NT keys): one wavefront per
+// workgroup takes 32 queries of one (sequence, head) and keeps their scores
+// against every key in registers, so K is multiplied once, the softmax sum
+// is taken against the final maximum, and there is no V^T copy: K and V rows
+// go to LDS in one burst of direct loads and V's fragments are gathered from
+// its rows, 16 bits at a time. The same scores, exponentials and roundings as
+// the kernel above.
+//
+// What bounds it: the latency of one wavefront (load, products, softmax,
+// products), so the workgroups are as small as they can be. 77 tokens of 32
+// heads of 64: 14.6 + 3.0 us with the two-pass kernel (32 workgroups of two
+// wavefronts) and its V^T copy, 6.8 us here (96 of one).
+template <int HD, int OUT_MODE, int NT>
+__global__ __launch_bounds__(64) void attention_short_kernel(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
+    const uint16_t* __restrict__ v, void* __restrict__ out, int64_t T, int group, int q_heads,
+    int64_t q_stride, int64_t kv_stride, int64_t out_stride, int64_t window, float scale,
+    int n_qb) {
+    using L = AttnTile<HD, 1>;
+    constexpr bool POW2 = HD == 64;
+    constexpr int TILE = 32 * L::KRB;  // bytes of a 32-key tile of K or V
+    extern __shared__ __attribute__((aligned(1024))) char lds[];  // K tiles, then V tiles
+    const int lane = threadIdx.x;
+    const int c = lane & 31, hl = lane >> 5;
+    const int qb = n_qb - 1 - (int)blockIdx.x % n_qb;
+    const int h = ((int)blockIdx.x / n_qb) % q_heads;
+    const int64_t b = (int)blockIdx.x / n_qb / q_heads;
+    const int64_t kvo = b * T * kv_stride + (int64_t)(h / group) * HD;
+    const uint32_t bytes = (uint32_t)(((T - 1) * kv_stride + HD) * 2);
+    const __amdgpu_buffer_rsrc_t rsk = make_rsrc(k + kvo, bytes);  // keys >= T load as zero
+    const __amdgpu_buffer_rsrc_t rsv = make_rsrc(v + kvo, bytes);
+    const int T32 = (int)T, win = window > 0 ? (int)window : T32;
+    const int q0 = 32 * qb, qq = q0 + c;
+    // Tiles with a visible key: t0 .. t1 - 1.
+    const int t1 = qb + 1, klo = q0 - win + 1, t0 = klo > 0 ? klo >> 5 : 0;
+
+    auto load = [&](__amdgpu_buffer_rsrc_t r, char* dst, uint32_t off) {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            r, (__attribute__((address_space(3))) void*)dst, 16, off, 0, 0, 0);
+    };
+    for (int t = t0; t < t1; ++t)
+#pragma unroll
+        for (int p = 0; p < 32 / L::KRPI; ++p) {
+            const int row = p * L::KRPI + lane / L::KCH;
+            const int ch = (lane % L::KCH) ^ ((row >> L::KSWZ) & (L::KCH - 1));
+            const uint32_t off = (uint32_t)((32 * t + row) * kv_stride * 2);
+            char* dst = lds + t * TILE + p * 1024;
+            load(rsk, dst, off + ch * 16);
+            load(rsv, dst + NT * TILE, off + (lane % L::KCH) * 16);
+        }
+    u32x4_t qf[HD / 16];
+    {
+        const uint16_t* qrow = q + (b * T + qq) * q_stride + (int64_t)h * HD + 8 * hl;
+#pragma unroll
+        for (int s = 0; s < HD / 16; ++s)
+            qf[s] = qq < T32 ? *(const u32x4_t*)(qrow + 16 * s) : u32x4_t{0u, 0u, 0u, 0u};
+    }
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));
+    asm volatile("" ::: "memory");
+
+    // Scores (rounded; for POW2 the scale is folded into the exponent's
+    // multiplier, as above) and their maximum.
+    constexpr float kLog2e = 1.4426950408889634f;
+    const float sl = POW2 ? scale * kLog2e : kLog2e;
+    auto round_pairs = [](f32x16_t& x) {
+#pragma unroll
+        for (int i = 0; i < 16; i += 2) {
+            const uint32_t p = bf16x2_rne(x[i], x[i + 1]);
+            x[i] = __uint_as_float(p << 16);
+            x[i + 1] = __uint_as_float(p & 0xFFFF0000u);
+        }
+    };
+    const int krow = key_perm(c);
+    const int kswz = (krow >> L::KSWZ) & (L::KCH - 1);
+    f32x16_t acc[NT];
+    float m = -INFINITY;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        if (t < t0 || t >= t1) continue;
+        f32x16_t x = {};
+        const char* rowp = lds + t * TILE + krow * L::KRB;
+#pragma unroll
+        for (int s = 0; s < HD / 16; ++s) {
+            const u32x4_t kf = *(const u32x4_t*)(rowp + (((2 * s + hl) ^ kswz) * 16));
+            x = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, kf),
+                                                        __builtin_bit_cast(bf16x8_t, qf[s]), x,
+                                                        0, 0, 0);
+        }
+        round_pairs(x);
+        if (!POW2) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) x[i] = x[i] * scale;
+            round_pairs(x);
+        }
+        if (t == t1 - 1 || 32 * t + win <= q0 + 31) {  // the diagonal, a window's edge
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const int key = 32 * t + key_perm(8 * (i / 4) + 4 * hl + (i % 4));
+                x[i] = key <= qq && key < T32 && key + win > qq ? x[i] : -INFINITY;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i) m = fmaxf(m, x[i]);
+        acc[t] = x;
+    }
+    {
+        const u32x2_t sw = swap32(__float_as_uint(m));
+        m = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+    }
+    float lsum = 0.0f;
+    const float nm0 = m == -INFINITY ? -INFINITY : -m * sl;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        if (t < t0 || t >= t1) continue;
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+            lsum = lsum + __builtin_amdgcn_exp2f(fmaf(acc[t][i], sl, nm0));
+    }
+    {
+        const u32x2_t sw = swap32(__float_as_uint(lsum));
+        lsum = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
+    }
+    const float nm = lsum > 0.0f ? nm0 - __builtin_amdgcn_logf(lsum) : -INFINITY;
+
+    constexpr int ND = HD / 32;
+    f32x16_t o[ND];
+#pragma unroll
+    for (int n = 0; n < ND; ++n) o[n] = f32x16_t{};
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        if (t < t0 || t >= t1) continue;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            u32x4_t pa;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                pa[e] = bf16x2_rne(
+                    __builtin_amdgcn_exp2f(fmaf(acc[t][8 * j + 2 * e], sl, nm)),
+                    __builtin_amdgcn_exp2f(fmaf(acc[t][8 * j + 2 * e + 1], sl, nm)));
+            // B of P V: dim 32 n + c of keys 32 t + 16 j + 8 hl .. + 7.
+            const uint16_t* vp =
+                (const uint16_t*)(lds + (NT + t) * TILE) + (16 * j + 8 * hl) * HD + c;
+#pragma unroll
+            for (int n = 0; n < ND; ++n) {
+                u32x4_t vb;
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    vb[e] = (uint32_t)vp[(2 * e) * HD + 32 * n] |
+                            ((uint32_t)vp[(2 * e + 1) * HD + 32 * n] << 16);
+                o[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                    __builtin_bit_cast(bf16x8_t, pa), __builtin_bit_cast(bf16x8_t, vb), o[n], 0,
+                    0, 0);
+            }
+        }
+    }
+#pragma unroll
+    for (int n = 0; n < ND; ++n)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const int qrow = q0 + 8 * (i / 4) + 4 * hl + (i % 4);
+            if (qrow >= T32) continue;
+            const uint32_t bits = bf16_bits_rne(o[n][i]);
+            const int64_t off = (b * T + qrow) * out_stride + (int64_t)h * HD + 32 * n + c;
+            if (OUT_MODE == NCM_OUT_BF16)
+                ((uint16_t*)out)[off] = (uint16_t)bits;
+            else
+                ((float*)out)[off] = __uint_as_float(bits << 16);
+        }
+}
+
+}  // namespace
+
 int64_t attention_vt_padded(int64_t seq_len) { return (seq_len + kBk - 1) / kBk * kBk; }
 
 size_t attention_workspace_bytes(int64_t batch, int64_t seq_len, int kv_heads, int head_dim) {
@@ -565,25 +742,72 @@ namespace {
 template <int HD>
 constexpr int attn_waves() { return HD == 64 ? 2 : 4; }
 
-template <int HD, int MASK>
-hipError_t launch_attn_hd(const uint16_t* q, const uint16_t* k, const uint16_t* v, void* out,
-                          int64_t batch, int64_t T, int hq, int hkv, int64_t q_stride,
-                          int64_t kv_stride, int64_t out_stride, int64_t window, SegArgs sa,
-                          int out_mode, uint16_t* vt, hipStream_t stream) {
+// Query blocks (over all heads and sequences) up to which a causal launch
+// gives each its own workgroup: they are then resident together and the
+// longest sets the time, where pairing a long with a short one would add the
+// two up. Measured, paired -> unpaired: head_dim 64, 32 heads, T = 512 / 1024 27 ->
+// 22 / 42 -> 37 us (256 / 512 blocks), no difference at 576; head_dim 128, 32 heads,
+// T = 512 / 1024 45 -> 33 / 67 -> 55 us (128 / 256 blocks), slower at 512.
+template <int HD>
+constexpr int64_t unpaired_groups() { return HD == 64 ? 512 : 384; }
+// The short kernel's range: sequences whose scores fit the registers, and
+// workgroups that fit the chip in about one round (each holds all of its K and
+// V in LDS: 32 or 64 KB at head_dim 64, 64 or 128 KB at 128). Measured, the
+// kernels above -> here: head_dim 64, 32 heads, T = 77 / 256 16.3 -> 10.2 / 20.3 -> 10.1
+// us a call, 4 x 256 (1024 workgroups) 21.2 -> 20.4; head_dim 128, T = 256 34 -> 14, 4 x
+// 160 (640) 29.5 -> 27.6, but 4 x 200 (896) 33.6 -> 39.4.
+constexpr int64_t kShortKeys = 256;
+template <int HD>
+constexpr int64_t short_groups() { return HD == 64 ? 1024 : 640; }
+
+template <int HD, int OUT_MODE, int NT>
+hipError_t launch_attn_short_t(const uint16_t* q, const uint16_t* k, const uint16_t* v, void* out,
+                               int64_t batch, int64_t T, int hq, int hkv, int64_t q_stride,
+                               int64_t kv_stride, int64_t out_stride, int64_t window,
+                               hipStream_t stream) {
+    auto kern = attention_short_kernel<HD, OUT_MODE, NT>;
+    constexpr int lds = 2 * NT * 32 * HD * 2;
+    static const hipError_t attr = hipFuncSetAttribute(
+        (const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (attr != hipSuccess) return attr;
+    const int n_qb = (int)((T + 31) / 32);
+    hipLaunchKernelGGL(kern, dim3((unsigned)(n_qb * hq * batch)), dim3(64), lds, stream, q, k, v,
+                       out, T, hq / hkv, hq, q_stride, kv_stride, out_stride, window,
+                       1.0f / sqrtf((float)HD), n_qb);
+    return hipGetLastError();
+}
+
+template <int HD>
+hipError_t launch_attn_short(const uint16_t* q, const uint16_t* k, const uint16_t* v, void* out,
+                             int64_t batch, int64_t T, int hq, int hkv, int64_t q_stride,
+                             int64_t kv_stride, int64_t out_stride, int64_t window, int out_mode,
+                             hipStream_t st) {
+#define NCM_SHORT(MODE, NT)                                                                   \
+    return launch_attn_short_t<HD, MODE, NT>(q, k, v, out, batch, T, hq, hkv, q_stride,       \
+                                             kv_stride, out_stride, window, st)
+    if (out_mode == NCM_OUT_BF16) {
+        if (T <= 128) NCM_SHORT(NCM_OUT_BF16, 4);
+        NCM_SHORT(NCM_OUT_BF16, 8);
+    }
+    if (T <= 128) NCM_SHORT(NCM_OUT_BF16_F32, 4);
+    NCM_SHORT(NCM_OUT_BF16_F32, 8);
+#undef NCM_SHORT
+}
+
+template <int HD, int MASK, bool PAIR>
+hipError_t launch_attn_blocks(const uint16_t* q, const uint16_t* k, void* out, int64_t batch,
+                              int64_t T, int hq, int hkv, int64_t q_stride, int64_t kv_stride,
+                              int64_t out_stride, int64_t window, SegArgs sa, int out_mode,
+                              uint16_t* vt, hipStream_t stream) {
     constexpr int NWV = attn_waves<HD>();
     const int64_t Tp = attention_vt_padded(T);
-    hipLaunchKernelGGL(attention_vt_kernel,
-                       dim3((unsigned)(Tp / 64), (unsigned)(hkv * HD / 64), (unsigned)batch),
-                       dim3(256), 0, stream, v, vt, T, Tp, kv_stride, (int64_t)hkv * HD);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
     const int64_t nqb = (T + 32 * NWV - 1) / (32 * NWV);
-    const int n_xb = (int)(MASK == 0 ? (nqb + 1) / 2 : nqb);
+    const int n_xb = (int)(PAIR ? (nqb + 1) / 2 : nqb);
     const dim3 grid((unsigned)((int64_t)n_xb * hq * batch));
     const float scale = 1.0f / sqrtf((float)HD);
     const int group = hq / hkv;
-    auto kb16 = attention_bf16_kernel<HD, NCM_OUT_BF16, MASK, NWV>;
-    auto kf32 = attention_bf16_kernel<HD, NCM_OUT_BF16_F32, MASK, NWV>;
+    auto kb16 = attention_bf16_kernel<HD, NCM_OUT_BF16, MASK, NWV, PAIR>;
+    auto kf32 = attention_bf16_kernel<HD, NCM_OUT_BF16_F32, MASK, NWV, PAIR>;
     size_t shm = 0;
     if constexpr (attn_dyn_lds<HD>()) {
         shm = AttnTile<HD, NWV>::LDS;
@@ -606,6 +830,32 @@ hipError_t launch_attn_hd(const uint16_t* q, const uint16_t* k, const uint16_t* 
         hipLaunchKernelGGL(kf32, grid, dim3(64 * NWV), shm, stream, q, k, vt, out, T, Tp, group,
                            hkv, q_stride, kv_stride, out_stride, window, scale, sa, n_xb);
     return hipGetLastError();
+}
+
+template <int HD, int MASK>
+hipError_t launch_attn_hd(const uint16_t* q, const uint16_t* k, const uint16_t* v, void* out,
+                          int64_t batch, int64_t T, int hq, int hkv, int64_t q_stride,
+                          int64_t kv_stride, int64_t out_stride, int64_t window, SegArgs sa,
+                          int out_mode, uint16_t* vt, hipStream_t stream) {
+    constexpr int NWV = attn_waves<HD>();
+    if (MASK == 0 && T <= kShortKeys && (T + 31) / 32 * hq * batch <= short_groups<HD>())
+        return launch_attn_short<HD>(q, k, v, out, batch, T, hq, hkv, q_stride, kv_stride,
+                                     out_stride, window, out_mode, stream);
+    const int64_t Tp = attention_vt_padded(T);
+    hipLaunchKernelGGL(attention_vt_kernel,
+                       dim3((unsigned)(Tp / 64), (unsigned)(hkv * HD / 64), (unsigned)batch),
+                       dim3(256), 0, stream, v, vt, T, Tp, kv_stride, (int64_t)hkv * HD);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    if constexpr (MASK == 0) {
+        const int64_t nqb = (T + 32 * NWV - 1) / (32 * NWV);
+        if (nqb * hq * batch > unpaired_groups<HD>())
+            return launch_attn_blocks<HD, 0, true>(q, k, out, batch, T, hq, hkv, q_stride,
+                                                   kv_stride, out_stride, window, sa, out_mode,
+                                                   vt, stream);
+    }
+    return launch_attn_blocks<HD, MASK, false>(q, k, out, batch, T, hq, hkv, q_stride, kv_stride,
+                                               out_stride, window, sa, out_mode, vt, stream);
 }
 
 }  // namespace
