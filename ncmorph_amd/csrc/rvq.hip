@@ -922,6 +922,197 @@ __global__ __launch_bounds__(256) void rvq_rescore_kernel(RowArgs a) {
     finish_row<NCH, KEEP_D, PAIR>(a, row, b, best_row, have_row, st.unorm2, lane, D, ch);
 }
 
+// ------------------------------------------------ every level in one launch
+
+// The encode of a few rows with every level at full resolution (all strides
+// 1): rows are then independent of each other, so one workgroup carries its
+// rows through every level without leaving the chip, and each level's search
+// is exact from the start: every code's distance in the fixed order (the
+// bits of dot_fixed), lowest index at the minimum. Its eight wavefronts split
+// the codes, 64 at a time: a lane accumulates its elements of 64 dot products
+// and the xor butterfly runs transposed (at each step a lane pair splits the
+// codes it still holds), which leaves code 64 g + j's sum in lane j after 63
+// exchanges instead of 6 per code.
+//
+// Bound: the latency of a level (the code rows' loads, the products, the
+// reductions), which with few rows is below that of the distance GEMM's and
+// the rescore's launches. Measured at 128 rows, d 256, 512 codes, four levels: 50
+// us for the 10 launches, 29.5 us for this one.
+constexpr int kFlatWaves = 8;
+
+// v[i] summed with its partner's over lane bit OFF; the lower side keeps the
+// first half of the values, the upper side the second half.
+template <int OFF, int N>
+__device__ __forceinline__ void halve_sum(float (&v)[N], int lane) {
+    constexpr int H = OFF;
+    if constexpr (OFF == 32 || OFF == 16) {
+#pragma unroll
+        for (int i = 0; i < H; ++i) {
+            const uint32_t a = __float_as_uint(v[i]), b = __float_as_uint(v[i + H]);
+            if constexpr (OFF == 32) {
+                auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+                v[i] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+            } else {
+                auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+                v[i] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+            }
+        }
+    } else {
+        const bool up = (lane & OFF) != 0;
+#pragma unroll
+        for (int i = 0; i < H; ++i) {
+            const float send = up ? v[i] : v[i + H];
+            const float keep = up ? v[i + H] : v[i];
+            float recv;
+            if constexpr (OFF == 8)
+                recv = __uint_as_float(dpp_u32<kDppRor8>(__float_as_uint(send)));
+            else if constexpr (OFF == 2)
+                recv = __uint_as_float(dpp_u32<kDppXor2>(__float_as_uint(send)));
+            else if constexpr (OFF == 1)
+                recv = __uint_as_float(dpp_u32<kDppXor1>(__float_as_uint(send)));
+            else
+                recv = __shfl_xor(send, OFF);
+            v[i] = keep + recv;
+        }
+    }
+}
+
+struct FlatArgs {
+    const float* x;
+    const uint16_t* cb;  // [levels, v, d]
+    const float* csq;    // [levels, v]
+    const int32_t* force_codes;
+    int32_t* codes;  // [b, levels t]
+    float* recon;    // nullable
+    int64_t t, d, v, rows;
+    int levels;
+};
+
+template <int NCH>
+__global__ __launch_bounds__(64 * kFlatWaves) void rvq_flat_kernel(FlatArgs a) {
+    constexpr int kBatch = 64 / NCH;  // code rows in flight
+    __shared__ float red_d[2][kFlatWaves];
+    __shared__ int32_t red_k[2][kFlatWaves];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t row = blockIdx.x;
+    const int64_t d = a.d, bb = row / a.t, tt = row - bb * a.t;
+    RowVec<NCH> x, D, u;
+    load_f32_row<NCH>(a.x + row * d, d, lane, x);
+    // A lane's offsets in a code row; past the row it loads zeros, whose
+    // products with u's zeros there change no sum.
+    uint32_t off[NCH];
+#pragma unroll
+    for (int m = 0; m < NCH; ++m)
+        off[m] = lane_chunk_valid(d, m, lane) ? (uint32_t)(m * 512 + 8 * lane) : kOobOffset;
+#pragma unroll
+    for (int m = 0; m < NCH; ++m)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) D.v[m][e] = 0.0f;
+    for (int l = 0; l < a.levels; ++l) {
+        bool finite = true;
+#pragma unroll
+        for (int m = 0; m < NCH; ++m)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                u.v[m][e] = x.v[m][e] - D.v[m][e];
+                finite = finite && fabsf(u.v[m][e]) < INFINITY;
+            }
+        const uint16_t* cbl = a.cb + (int64_t)l * a.v * d;
+        const float* csql = a.csq + (int64_t)l * a.v;
+        const __amdgpu_buffer_rsrc_t rsc = make_rsrc(cbl, (uint32_t)(a.v * d * 2));
+        float best = INFINITY;
+        int32_t code = 0x7FFFFFFF;
+        auto take = [&](float od, int32_t oc) {
+            if (od < best || (od == best && oc < code)) {
+                best = od;
+                code = oc;
+            }
+        };
+        for (int64_t g0 = 64 * wave; g0 < a.v; g0 += 64 * kFlatWaves) {
+            float dots[64];
+#pragma unroll
+            for (int c0 = 0; c0 < 64; c0 += kBatch) {
+                u32x2_t p[kBatch][NCH];
+#pragma unroll
+                for (int j = 0; j < kBatch; ++j) {
+                    const int64_t k = g0 + c0 + j < a.v ? g0 + c0 + j : a.v - 1;
+#pragma unroll
+                    for (int m = 0; m < NCH; ++m)
+                        p[j][m] = __builtin_amdgcn_raw_buffer_load_b64(rsc, off[m],
+                                                                       (int)(k * d * 2), 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int j = 0; j < kBatch; ++j) {
+                    float acc = 0.0f;
+#pragma unroll
+                    for (int m = 0; m < NCH; ++m) {
+                        acc = __builtin_fmaf(u.v[m][0], bf16_lo_to_f32(p[j][m][0]), acc);
+                        acc = __builtin_fmaf(u.v[m][1], bf16_hi_to_f32(p[j][m][0]), acc);
+                        acc = __builtin_fmaf(u.v[m][2], bf16_lo_to_f32(p[j][m][1]), acc);
+                        acc = __builtin_fmaf(u.v[m][3], bf16_hi_to_f32(p[j][m][1]), acc);
+                    }
+                    dots[c0 + j] = acc;
+                }
+            }
+            halve_sum<32>(dots, lane);
+            halve_sum<16>(dots, lane);
+            halve_sum<8>(dots, lane);
+            halve_sum<4>(dots, lane);
+            halve_sum<2>(dots, lane);
+            halve_sum<1>(dots, lane);
+            const int64_t k = g0 + lane;
+            if (k < a.v) {
+                const float dist = __builtin_fmaf(-2.0f, dots[0], csql[k]);
+                take(dist, (int32_t)k);
+            }
+        }
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1)
+            take(__shfl_xor(best, off), __shfl_xor(code, off));
+        if (lane == 0) {
+            red_d[l & 1][wave] = best;
+            red_k[l & 1][wave] = code;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < kFlatWaves; ++w) take(red_d[l & 1][w], red_k[l & 1][w]);
+        // A row that is not finite has no code under the rescore's threshold.
+        if (__ballot(!finite)) code = 0x7FFFFFFF;
+        const int64_t ci = (bb * a.levels + l) * a.t + tt;
+        if (threadIdx.x == 0) a.codes[ci] = code;
+        int32_t k = a.force_codes ? a.force_codes[ci] : code;
+        k = k < 0 ? 0 : (k >= a.v ? (int32_t)(a.v - 1) : k);
+        add_bf16_row<NCH>(cbl + (int64_t)k * d, d, lane, D);
+    }
+    if (a.recon && wave == 0) {
+        float* dst = a.recon + row * d;
+#pragma unroll
+        for (int m = 0; m < NCH; ++m)
+            if (lane_chunk_valid(d, m, lane))
+                *(f32x4_t*)(dst + m * 256 + 4 * lane) =
+                    f32x4_t{D.v[m][0], D.v[m][1], D.v[m][2], D.v[m][3]};
+    }
+}
+
+// Where rvq_flat_kernel takes an encode: full-resolution levels, no gaps or
+// counts asked for (they describe the rescore), a workgroup for every row at
+// once (one per CU), and few enough codes: a row's workgroup reads all of
+// them, a wavefront's loads taking 256 elements of each. Measured, three
+// levels, the launches below -> this one: 8 .. 256 rows of d 128 or 256 with 512
+// codes 32-35 -> 22 us, 1024 codes 34-37 -> 33-34 us, of d 512 with 512 codes
+// 37-40 -> 33-34 us; but d 1024, 512 codes 48 -> 53-79 us, d 256, 2048 codes 36 -> 60
+// us, and 512 rows of d 256, 512 codes 37 -> 44 us.
+constexpr int64_t kFlatMaxRows = 256;
+constexpr int64_t kFlatMaxLoads = 1024;  // codes x 256-element pieces of a code
+
+static bool flat_fits(int64_t rows, int64_t d, int64_t v, const int32_t* strides, bool wants_gap,
+                      bool wants_counts) {
+    return strides[0] == 1 && !wants_gap && !wants_counts && rows <= kFlatMaxRows && d <= 512 &&
+           v * ((d + 255) / 256) <= kFlatMaxLoads;
+}
+
 // ------------------------------------------------------------ host side
 
 // Distance GEMM tiles (codes x rows), all loading global -> LDS directly
@@ -1179,8 +1370,18 @@ int rvq_encode_ws(hipStream_t st, void* ws, size_t ws_bytes, const float* x, int
     // D_{l+1} (coarse reconstruction) is written by level l into dbuf[(l+1)&1].
     float* dbuf[2] = {(float*)(W + lay.d0), (float*)(W + lay.d1)};
 
-    const SetupArgs sa{csq, v, levels, cmax, fcount};
     hipError_t e = hipSuccess;
+    if (flat_fits(b * t, d, v, strides, gap != nullptr, n_flagged || counts)) {
+        const FlatArgs fa{x, codebooks, csq, force_codes, codes, recon, t, d, v, b * t,
+                          (int)levels};
+        const dim3 grid((unsigned)(b * t)), block(64 * kFlatWaves);
+        if (d <= 256)
+            hipLaunchKernelGGL(rvq_flat_kernel<1>, grid, block, 0, st, fa);
+        else
+            hipLaunchKernelGGL(rvq_flat_kernel<2>, grid, block, 0, st, fa);
+        return hipGetLastError() == hipSuccess ? NCM_OK : NCM_E_HIP;
+    }
+    const SetupArgs sa{csq, v, levels, cmax, fcount};
     if (jmax == 0) {
         hipLaunchKernelGGL(rvq_setup_kernel, dim3((unsigned)levels), dim3(kSetupThreads), 0, st,
                            sa);
