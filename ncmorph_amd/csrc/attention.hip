@@ -747,9 +747,15 @@ constexpr int attn_waves() { return HD == 64 ? 2 : 4; }
 // longest sets the time, where pairing a long with a short one would add the
 // two up. Measured, paired -> unpaired: head_dim 64, 32 heads, T = 512 / 1024 27 ->
 // 22 / 42 -> 37 us (256 / 512 blocks), no difference at 576; head_dim 128, 32 heads,
-// T = 512 / 1024 45 -> 33 / 67 -> 55 us (128 / 256 blocks), slower at 512.
+// T = 512 / 1024 45 -> 33 / 67 -> 55 us (128 / 256 blocks), slower at 512. Past a
+// block or so per CU that takes whole (sequence, kv head) groups on every XCD:
+// a run that ends inside one gives an XCD its longest blocks and the next XCD
+// its shortest (head_dim 64, 12 groups, 700 keys, 396 blocks: 33.1 -> 34.4 us; 6
+// and 12 groups of 288 blocks 42 -> 37 and 27.6 -> 23.7).
 template <int HD>
-constexpr int64_t unpaired_groups() { return HD == 64 ? 512 : 384; }
+constexpr int64_t unpaired_groups(int64_t kv_groups) {
+    return kv_groups % 8 != 0 ? 288 : (HD == 64 ? 512 : 384);
+}
 // The short kernel's range: sequences whose scores fit the registers, and
 // workgroups that fit the chip in about one round (each holds all of its K and
 // V in LDS: 32 or 64 KB at head_dim 64, 64 or 128 KB at 128). Measured, the
@@ -849,7 +855,7 @@ hipError_t launch_attn_hd(const uint16_t* q, const uint16_t* k, const uint16_t* 
     if (e != hipSuccess) return e;
     if constexpr (MASK == 0) {
         const int64_t nqb = (T + 32 * NWV - 1) / (32 * NWV);
-        if (nqb * hq * batch > unpaired_groups<HD>())
+        if (nqb * hq * batch > unpaired_groups<HD>(hkv * batch))
             return launch_attn_blocks<HD, 0, true>(q, k, out, batch, T, hq, hkv, q_stride,
                                                    kv_stride, out_stride, window, sa, out_mode,
                                                    vt, stream);
