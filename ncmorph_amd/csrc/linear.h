@@ -8,7 +8,11 @@ namespace ncm {
 
 // Tile configuration chosen for an M x N output (see the table in
 // linear.hip); a valid `forced` index overrides the choice.
-int linear_tile_config(int64_t M, int64_t N, int64_t K, int forced);
+int linear_tile_config(int64_t M, int64_t N, int forced);
+// The automatic choice's tiles besides configurations 0 (256x256) and 1
+// (128x128), and its cost: 100 is a full round of 256x256 tiles.
+constexpr int kTile128x256 = 16, kTile64x128 = 17;
+int64_t linear_tile_cost(int64_t M, int64_t N, int* tile);
 
 hipError_t launch_linear(const uint16_t* x, const uint16_t* w, const uint16_t* bias, void* y,
                          int64_t M, int64_t K, int64_t N, int out_mode, int config,
@@ -40,10 +44,9 @@ hipError_t launch_linear_rope64(const uint16_t* x, const uint16_t* w, const uint
 
 // Rows past the last full 256-row tile that launch_linear,
 // launch_linear_residual and launch_linear_swiglu (automatic tile choice)
-// hand to linear_tail.hip, or 0: M % 256 when it is at most 64, the
-// 256 x 256 tile is chosen for M and for M - M % 256, K % 2048 == 0,
-// N % 16 == 0, and the partial row tile would cost the whole chip an extra
-// round (N: the weight's rows).
+// hand to linear_tail.hip, or 0: M % 256 when it is at most 64, K % 2048 ==
+// 0, N % 16 == 0, the 256 x 256 tile is chosen for the other rows, and the two
+// launches cost less than the best tile over all rows (N: the weight's rows).
 int64_t linear_tail_rows(int64_t M, int64_t N, int64_t K);
 // The R rows of such a tail (x, y, residual pointing at its first row):
 // out_mode / bias / residual as launch_linear(_residual); swiglu: N is the

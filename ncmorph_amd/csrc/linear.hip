@@ -228,6 +228,12 @@ using Lin12 = GemmShape<128, 128, 64, 2, 2, 2, 5, true, 4>;
 using Lin13 = GemmShape<256, 128, 64, 4, 2, 2, 5, true, 3>;
 using Lin14 = GemmShape<256, 256, 64, 4, 2, 2, 8, true, 2, false, 1, -1, 2>;
 using Lin15 = GemmShape<256, 128, 64, 4, 2, 2, 8, true, 3>;
+// The automatic choice's own (no index):
+//  kTile128x256  128x256x64, 8 waves (64x64), as 5 otherwise
+//  kTile64x128   64x128x64, 4 waves (32x64), 4 stages: one workgroup per CU, taken
+//                for up to one round (600 x 8192 x 2048: 36 us; 42 with 3 stages)
+using Lin128x256 = GemmShape<128, 256, 64, 2, 4, 2, 8, true, 3, false, 1, -1, -1, true>;
+using Lin64x128 = GemmShape<64, 128, 64, 2, 2, 2, 8, true, 4, false, 1, -1, -1, true>;
 constexpr int kLinConfigs = 16;
 
 // fp32 linear: 128x128x32 (128-byte rows), 4 waves, DMA, SCHED 5, two
@@ -235,20 +241,45 @@ constexpr int kLinConfigs = 16;
 // rate, so this tile is MFMA-bound with a wide margin.
 using LinF32 = GemmShape<128, 128, 32, 2, 2, 2, 5, true, 2, true>;
 
-int linear_tile_config(int64_t M, int64_t N, int64_t K, int forced) {
+// The tile of an M x N product: the least number of rounds of the 256 CUs
+// times the time of a round, relative to a round of 256x256 tiles. Measured (K 576
+// .. 8192, M 70 .. 6000, N 2048 .. 151936), a round of 256x256 at K 2048 takes 45 us,
+// of 128x256 24 and in products of many rounds 27, of 128x128 14-18, of 64x128 11.
+// All four sum in the same order, so the choice does not change a bit.
+//
+// Where the choice falls, 256x256 (three quarters of a round or more), 256x128 or
+// 128x128 with two stages -> here, us: 77 rows of 128256 x 2048 164 -> 136 and of
+// 151936 x 1024 120 -> 81 (256-row tiles multiply 179 rows of padding), 300 rows
+// 253 -> 220 and 175 -> 148 (384 rows instead of 512), 700 of 28672 x 4096 185 ->
+// 153, 1500 of 16384 x 2048 113 -> 95 (3 rounds of halves for 2), 300 of 3072 x 2048
+// 15.4 -> 12.1, 1000 of 2048 x 8192 48 -> 40.
+struct TileCost {
+    int bm, bn, cost, tile;
+};
+constexpr TileCost kTiles[] = {{256, 256, 100, 0},
+                               {128, 256, 59, kTile128x256},
+                               {128, 128, 35, 1},
+                               {64, 128, 25, kTile64x128}};
+constexpr int64_t kTileCus = 256;
+
+int64_t linear_tile_cost(int64_t M, int64_t N, int* tile) {
+    int64_t best = INT64_MAX;
+    for (const TileCost& t : kTiles) {
+        const int64_t n = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+        const int64_t c = ((n + kTileCus - 1) / kTileCus) * t.cost;
+        if (c < best) {
+            best = c;
+            *tile = t.tile;
+        }
+    }
+    return best;
+}
+
+int linear_tile_config(int64_t M, int64_t N, int forced) {
     if (forced >= 0 && forced < kLinConfigs) return forced;
-    const int64_t cus = 256;
-    auto tiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
-    // 256x256 with 8 waves when it fills at least three quarters of the
-    // CUs; 128x128 with four LDS stages when that gives at most one tile per
-    // CU (latency-bound: deeper prefetch pays); 256x128 with three stages
-    // when its tiles fill the CUs about once or twice; else 128x128 with two
-    // stages (two workgroups per CU). All with direct-to-LDS loads.
-    // (Measured on the decoder's and the benchmark's shapes.)
-    if (tiles(256, 256) * 4 >= cus * 3) return 0;
-    if (tiles(128, 128) <= cus) return 1;
-    if (tiles(256, 128) * 4 >= cus * 3 && tiles(256, 128) <= 2 * cus) return 5;
-    return 2;
+    int tile = 0;
+    linear_tile_cost(M, N, &tile);
+    return tile;
 }
 
 hipError_t launch_linear(const uint16_t* x, const uint16_t* w, const uint16_t* bias, void* y,
@@ -275,7 +306,7 @@ hipError_t launch_linear(const uint16_t* x, const uint16_t* w, const uint16_t* b
                                       K, N, out_mode, false, stream);
         }
     }
-    switch (linear_tile_config(M, N, K, config)) {
+    switch (linear_tile_config(M, N, config)) {
         case 0: return launch_linear_s<Lin0>(x, w, bias, y, M, K, N, out_mode, stream);
         case 1: return launch_linear_s<Lin1>(x, w, bias, y, M, K, N, out_mode, stream);
         case 2: return launch_linear_s<Lin2>(x, w, bias, y, M, K, N, out_mode, stream);
@@ -291,7 +322,10 @@ hipError_t launch_linear(const uint16_t* x, const uint16_t* w, const uint16_t* b
         case 12: return launch_linear_s<Lin12>(x, w, bias, y, M, K, N, out_mode, stream);
         case 13: return launch_linear_s<Lin13>(x, w, bias, y, M, K, N, out_mode, stream);
         case 14: return launch_linear_s<Lin14>(x, w, bias, y, M, K, N, out_mode, stream);
-        default: return launch_linear_s<Lin15>(x, w, bias, y, M, K, N, out_mode, stream);
+        case 15: return launch_linear_s<Lin15>(x, w, bias, y, M, K, N, out_mode, stream);
+        case kTile128x256:
+            return launch_linear_s<Lin128x256>(x, w, bias, y, M, K, N, out_mode, stream);
+        default: return launch_linear_s<Lin64x128>(x, w, bias, y, M, K, N, out_mode, stream);
     }
 }
 
@@ -313,8 +347,8 @@ static hipError_t launch_linear_res_s(const uint16_t* x, const uint16_t* w, cons
 hipError_t launch_linear_residual(const uint16_t* x, const uint16_t* w, const uint16_t* bias,
                                   const float* residual, void* y, int64_t M, int64_t K,
                                   int64_t N, int out_mode, hipStream_t stream) {
-    // The automatic choice only: the K-sliced kernel, or configurations 0, 1,
-    // 2 and 5 with the tail rows of linear_tail_rows on the tail kernel.
+    // The automatic choice only: the K-sliced kernel, or a tile with the tail
+    // rows of linear_tail_rows on the tail kernel.
     if (linear_slice_fits(M, N, K))
         return launch_linear_slice(x, w, bias, residual, y, M, K, N, out_mode, stream);
     const int64_t r = linear_tail_rows(M, N, K);
@@ -327,11 +361,15 @@ hipError_t launch_linear_residual(const uint16_t* x, const uint16_t* w, const ui
         return launch_linear_tail(x + mm * K, w, bias, residual + mm * N,
                                   (char*)y + mm * N * esz, r, K, N, out_mode, false, stream);
     }
-    switch (linear_tile_config(M, N, K, -1)) {
+    switch (linear_tile_config(M, N, -1)) {
         case 0: return launch_linear_res_s<Lin0>(x, w, bias, residual, y, M, K, N, out_mode, stream);
         case 1: return launch_linear_res_s<Lin1>(x, w, bias, residual, y, M, K, N, out_mode, stream);
-        case 5: return launch_linear_res_s<Lin5>(x, w, bias, residual, y, M, K, N, out_mode, stream);
-        default: return launch_linear_res_s<Lin2>(x, w, bias, residual, y, M, K, N, out_mode, stream);
+        case kTile128x256:
+            return launch_linear_res_s<Lin128x256>(x, w, bias, residual, y, M, K, N, out_mode,
+                                                   stream);
+        default:
+            return launch_linear_res_s<Lin64x128>(x, w, bias, residual, y, M, K, N, out_mode,
+                                                  stream);
     }
 }
 

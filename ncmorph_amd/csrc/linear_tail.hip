@@ -267,14 +267,15 @@ int64_t linear_tail_rows(int64_t M, int64_t N, int64_t K) {
     if (r == 0 || r > kTailMaxRows || M < 256 || K % kTailKMultiple != 0 || N % 16 != 0 ||
         K > (int64_t)1 << 22)
         return 0;
-    const int64_t m_main = M - r;
-    if (linear_tile_config(M, N, K, -1) != 0 || linear_tile_config(m_main, N, K, -1) != 0)
-        return 0;
-    const int64_t cus = 256;
-    const int64_t tiles_n = (N + 255) / 256;
-    const int64_t rounds_main = ((m_main / 256) * tiles_n + cus - 1) / cus;
-    const int64_t rounds_all = ((m_main / 256 + 1) * tiles_n + cus - 1) / cus;
-    return rounds_all > rounds_main ? r : 0;
+    // Two launches when they cost less than the best tile over all rows; the
+    // rows before the tail on 256x256 tiles. The tail streams the whole
+    // weight: a round's tenth, and as much as a full round of 256x256 tiles for
+    // every 50000 columns (4096 columns of K 14336: 34 us against a round's 315;
+    // 28672 of K 4096: 59 against 88).
+    int tile_all, tile_main;
+    const int64_t all = linear_tile_cost(M, N, &tile_all);
+    const int64_t main = linear_tile_cost(M - r, N, &tile_main);
+    return tile_main == 0 && main + 10 + N / 500 < all ? r : 0;
 }
 
 hipError_t launch_linear_tail(const uint16_t* x, const uint16_t* w, const uint16_t* bias,
