@@ -212,7 +212,10 @@ static hipError_t launch_linear_s(const uint16_t* x, const uint16_t* w, const ui
 // 10: 128x128x128 (256-byte rows), 4 waves, DMA, SCHED 5, 2 stages
 // 11, 12, 13: as 0, 1 and 5 with SCHED 5 (all loads of a tile issued
 //     together at its start, fragment reads of a k-step as one group)
-using Lin0 = GemmShape<256, 256, 64, 4, 2, 2, 8, true, 2, false, 1, -1, -1, true>;
+// (0's 24: MFMAs of the last k-step issued before the K-tile barrier, of 32. The
+// 8192 x 4096 x 28672 and 4096 x 8192 x 2048 products take 1531 and 157 us at 16, 1489
+// and 150 at 20, 1469 and 149 at 24, 1466 and 149 at 28.)
+using Lin0 = GemmShape<256, 256, 64, 4, 2, 2, 8, true, 2, false, 1, 24, -1, true>;
 using Lin1 = GemmShape<128, 128, 64, 4, 2, 2, 8, true, 4, false, 1, -1, -1, true>;
 using Lin2 = GemmShape<128, 128, 64, 2, 2, 2, 4, true>;
 using Lin3 = GemmShape<256, 256, 32, 4, 2, 2, 6, true, 4>;

@@ -209,7 +209,7 @@ template <int EPI>
 static hipError_t launch_pair(const uint16_t* x, const uint16_t* w, const uint16_t* bias,
                               uint16_t* y, int64_t M, int64_t K, int64_t N, PairArgs pa,
                               hipStream_t st) {
-    using L0 = GemmShape<256, 256, 64, 4, 2, 2, 8, true, 2, false, 1, -1, -1, true>;
+    using L0 = GemmShape<256, 256, 64, 4, 2, 2, 8, true, 2, false, 1, 24, -1, true>;
     using L1 = GemmShape<128, 128, 64, 4, 2, 2, 8, true, 4, false, 1, -1, -1, true>;
     using L128x256 = GemmShape<128, 256, 64, 2, 4, 2, 8, true, 3, false, 1, -1, -1, true>;
     using L64x128 = GemmShape<64, 128, 64, 2, 2, 2, 8, true, 4, false, 1, -1, -1, true>;

@@ -1129,7 +1129,7 @@ static bool flat_fits(int64_t rows, int64_t d, int64_t v, const int32_t* strides
 using DistBig = GemmShape<256, 256, 64, 4, 2, 2, 8, true, 2, false, 1, -1, 2>;
 // DistBig on 16x16x32 MFMAs (its fragments take 48 more VGPRs: only with one
 // code tile per workgroup, when no per-row state lives through the main loop).
-using DistBig16 = GemmShape<256, 256, 64, 4, 2, 2, 8, true, 2, false, 1, -1, -1, true>;
+using DistBig16 = GemmShape<256, 256, 64, 4, 2, 2, 8, true, 2, false, 1, 24, -1, true>;
 using DistMid = GemmShape<256, 128, 64, 4, 2, 2, 8, true, 3, false, 1, -1, -1, true>;
 using DistSmall = GemmShape<128, 128, 64, 2, 2, 2, 8, true, 4>;
 using DistSmall2 = GemmShape<128, 128, 64, 2, 2, 2, 8, true, 2>;
