@@ -9,6 +9,7 @@
 
 #include "gemm_core.h"
 #include "linear.h"
+#include "linear_slice.h"
 
 namespace ncm {
 
@@ -239,10 +240,12 @@ using Lin128x256 = GemmShape<128, 256, 64, 2, 4, 2, 8, true, 3, false, 1, -1, -1
 using Lin64x128 = GemmShape<64, 128, 64, 2, 2, 2, 8, true, 4, false, 1, -1, -1, true>;
 constexpr int kLinConfigs = 16;
 
-// fp32 linear: 128x128x32 (128-byte rows), 4 waves, DMA, SCHED 5, two
-// stages (64 KB: two workgroups per CU). The fp32 MFMA has 1/16 of the bf16
-// rate, so this tile is MFMA-bound with a wide margin.
+// fp32 linear, four waves, DMA, two stages: 128x128x32 (128-byte rows, SCHED 5,
+// two workgroups per CU) and, where it is estimated to be faster, 64x64x32
+// (SCHED 8, four per CU). The fp32 MFMA has 1/16 of the bf16 rate and bounds
+// both; the small tile spreads 1.5 .. 3 rounds' worth of work more evenly.
 using LinF32 = GemmShape<128, 128, 32, 2, 2, 2, 5, true, 2, true>;
+using LinF32Small = GemmShape<64, 64, 32, 2, 2, 4, 8, true, 2, true>;
 
 // The tile of an M x N product: the least number of rounds of the 256 CUs
 // times the time of a round, relative to a round of 256x256 tiles. Measured (K 576
@@ -384,6 +387,8 @@ hipError_t launch_linear_f32(const float* x, const float* w, float* y, int64_t M
         l.M = M; l.K = K; l.N = N;
         return launch_linear_slice_f32(l, stream);
     }
+    if (f32_small_us(M, N, K) < f32_large_us(M, N, K))
+        return launch_linear_t<LinF32Small, NCM_OUT_F32, false>(x, w, nullptr, y, M, K, N, stream);
     return launch_linear_t<LinF32, NCM_OUT_F32, false>(x, w, nullptr, y, M, K, N, stream);
 }
 

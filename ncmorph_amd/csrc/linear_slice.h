@@ -184,18 +184,35 @@ constexpr int kSliceTileCount = sizeof(kSliceTiles) / sizeof(kSliceTiles[0]);
 
 // fp32: the matrix core is the bound (1/16 of the bf16 rate), so a tile is
 // priced in time: rounds of the CUs times the workgroup's MFMAs (0.22 us per
-// block of 16 x 16 outputs and iteration of its eight wavefronts) plus what
-// starting, summing and storing it takes, plus the launch. Fitted to M = 1 ..
-// 600 on the 135M and 0.5B checkpoints' projections, within 20% where the
-// weight stream is not the bound (200 rows, 576 x 576: 4.9 us + launch; 300 rows,
-// 4864 x 896: 35 us).
+// block of 16 x 16 outputs and iteration of its eight wavefronts, two on each
+// SIMD) plus what starting, summing and storing it takes, an eighth more past
+// one round (the operands then compete for the L2), plus the launch. Fitted to
+// M = 1 .. 13000, K = 384 .. 4864, within 15% where the weight stream is not the
+// bound (200 rows, 576 x 576: 5.1 us; 300 rows, 4864 x 896: 32 us; 4222 rows, 384 x
+// 1152: 49 us).
 inline double slice_f32_tile_us(const SliceTile& s, int64_t M, int64_t N, int64_t K) {
     const int64_t tiles =
         ((M + 16 * s.rb - 1) / (16 * s.rb)) * ((N + 16 * s.cb - 1) / (16 * s.cb));
-    // Two wavefronts a SIMD: its K tiles, in halves of an iteration.
     const double iters = 0.5 * (double)(((K + 31) / 32 + 3) / 4);
     const int blocks = s.rb * s.cb;
-    return 3.0 + (double)((tiles + 255) / 256) * (0.22 * blocks * iters + 1.3 + 0.3 * blocks);
+    const double round = 0.22 * blocks * iters + 1.3 + 0.3 * blocks;
+    const int64_t rounds = (tiles + 255) / 256;
+    return 3.0 + (rounds > 1 ? 1.12 * (double)rounds : 1.0) * round;
+}
+
+// The other fp32 tiles' time (linear.hip, vq_tok.hip): 128 x 128 tiles by their
+// rounds of the CUs (130 us for anything up to 256 tiles at K = 2048; from four
+// rounds on they overlap and take a tenth less), 64 x 64 tiles by those of the
+// fullest CU (within 10% over M = 64 .. 33000 at K = 384 .. 1536).
+inline double f32_large_us(int64_t M, int64_t N, int64_t K) {
+    const int64_t rounds = (((M + 127) / 128) * ((N + 127) / 128) + 255) / 256;
+    const double us = (double)rounds * (1.95 * ((K + 31) / 32) + 6.0);
+    return 3.0 + (rounds >= 4 ? 0.9 * us : us);
+}
+
+inline double f32_small_us(int64_t M, int64_t N, int64_t K) {
+    const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64);
+    return 6.5 + (double)((tiles + 255) / 256) * (0.5 * ((K + 31) / 32) + 0.6);
 }
 
 inline double slice_best_tile_f32(int64_t M, int64_t N, int64_t K, bool paired, int* tile) {

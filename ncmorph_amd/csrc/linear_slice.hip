@@ -330,14 +330,13 @@ hipError_t launch_linear_slice_rope64(const uint16_t* x, const uint16_t* w, cons
     return launch_slice<kRope>(tile, a, st);
 }
 
-// The 128 x 128 fp32 tiles take 2.03 us per 32-element K tile and round of the
-// CUs (130 us for anything up to 256 tiles at K = 2048).
+// Against the better of the two other fp32 tiles; a tenth in favour of this
+// kernel, whose fused epilogues save launches.
 bool linear_slice_f32_fits(int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || N <= 0 || K <= 0 || K > (int64_t)1 << 20) return false;
-    const int64_t big = ((M + 127) / 128) * ((N + 127) / 128);
-    const double big_us = (double)((big + 255) / 256) * (2.03 * ((K + 31) / 32) + 3.5) + 3.0;
     int tile;
-    return slice_best_tile_f32(M, N, K, false, &tile) < big_us;
+    const double us = slice_best_tile_f32(M, N, K, false, &tile);
+    return us < f32_large_us(M, N, K) && us < 1.1 * f32_small_us(M, N, K);
 }
 
 hipError_t launch_linear_slice_f32(const LinearF32& l, hipStream_t st) {

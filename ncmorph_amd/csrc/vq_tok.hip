@@ -34,10 +34,22 @@ namespace ncm {
 
 namespace {
 
-// 128 x 128 x 16 fp32 tile, 4 wavefronts of 64 x 64, two LDS stages (32 KB):
-// four workgroups per CU, 118 VGPRs (measured faster than 32-deep K tiles with
-// two workgroups per CU, deeper pipelines and 8-wavefront tiles).
-using VtTile = GemmShape<128, 128, 16, 2, 2, 4, 5, true, 2, true>;
+// fp32 tiles of four wavefronts, two LDS stages.
+//   VtSmall  64 x 64 x 32 (32 x 32 a wavefront), four workgroups per CU: the
+//            convolutions, whose 384 columns are few 128-column tiles. Phi of 96 /
+//            200 / 500 sequences 70 / 135 / 327 us (VtLarge or the K-sliced tiles,
+//            whichever the rule took) -> 60 / 102 / 241 us.
+//   VtWide   64 x 128 x 32 (32 x 64), three per CU: the searches, whose epilogue
+//            costs more per row. 1536 / 6144 rows against 4096 codes of 384: 58 /
+//            183 -> 48 / 178 us.
+//   VtLarge  128 x 128 x 16 (64 x 64), four per CU: searches of many tiles per
+//            CU. 32000 rows: 914 us on VtWide, 842 here.
+using VtSmall = GemmShape<64, 64, 32, 2, 2, 4, 8, true, 2, true>;
+using VtWide = GemmShape<64, 128, 32, 2, 2, 3, 8, true, 2, true>;
+using VtLarge = GemmShape<128, 128, 16, 2, 2, 4, 5, true, 2, true>;
+// 128 x 128 tiles per CU from which VtLarge takes a search (at 6 VtWide is 3%
+// faster, at 31 8% slower).
+constexpr int64_t kVtLargeTiles = 8 * 256;
 constexpr int kNT = 256;
 
 enum { kEpiStage = 0, kEpiPhi = 1, kEpiDist = 2 };
@@ -270,8 +282,8 @@ __attribute__((amdgpu_waves_per_eu(S::OCC, S::OCC))) void vt_gemm_kernel(
 }
 
 // The same product and epilogues on small tiles with K split over the
-// wavefronts (linear_slice.h), for products of too few 128 x 128 tiles: Phi of
-// 24 / 96 sequences is 39 / 150 of them and took 89 / 96 us, 26 / 75 here.
+// wavefronts (linear_slice.h), for products of too few tiles: Phi of 12 / 24 / 48
+// sequences 25 / 26 / 43 us on 64 x 64 tiles, 13 / 23 / 37 here.
 template <int RB, int CB, int NST, int EPI>
 __global__ __launch_bounds__(64 * kSliceWaves) void vt_slice_kernel(
     const float* __restrict__ a, int64_t lda, int64_t a_rows, const float* __restrict__ w,
@@ -439,33 +451,42 @@ hipError_t launch_vt_slice(int tile, const float* a, int64_t lda, int64_t a_rows
 #undef VT_SLICE
 }
 
-template <int EPI>
-hipError_t launch_vt_gemm(const float* a, int64_t lda, int64_t a_rows, const float* w, int64_t M,
+template <class S, int EPI>
+hipError_t launch_vt_tile(const float* a, int64_t lda, int64_t a_rows, const float* w, int64_t M,
                           int64_t K, int64_t N, const VtEpi& ep, hipStream_t st) {
-    using S = VtTile;
     auto kern = vt_gemm_kernel<S, EPI>;
-    static bool attr_set = false;
-    if (!attr_set) {
-        hipError_t e = hipFuncSetAttribute((const void*)kern,
-                                           hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           S::LDS_BYTES);
-        if (e != hipSuccess) return e;
-        attr_set = true;
-    }
-    if (M <= 0 || N <= 0) return hipSuccess;
+    static const hipError_t attr = hipFuncSetAttribute(
+        (const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, S::LDS_BYTES);
+    if (attr != hipSuccess) return attr;
     const int tiles_m = (int)((M + S::BM - 1) / S::BM);
     const int tiles_n = (int)((N + S::BN - 1) / S::BN);
-    // A round of 128 x 128 tiles: 2.6 us per 32 elements of K (96 us for up to
-    // 256 tiles at K = 1152).
-    const double big_us =
-        (double)(((int64_t)tiles_m * tiles_n + 255) / 256) * (2.6 * ((K + 31) / 32) + 4.0) + 3.0;
-    int tile = -1;
-    if (K > 0 && slice_best_tile_f32(M, N, K, false, &tile) < big_us)
-        return launch_vt_slice<EPI>(tile, a, lda, a_rows, w, M, K, N, ep, st);
     const int group_m = tiles_m < 4 ? tiles_m : 4;
     hipLaunchKernelGGL(kern, dim3(tiles_m * tiles_n), dim3(S::NT), S::LDS_BYTES, st, a, lda,
                        a_rows, w, M, K, N, tiles_n, group_m, ep);
     return hipGetLastError();
+}
+
+// The tile, by time: VtSmall or VtWide, priced by the tiles of the fullest CU,
+// against the K-sliced tiles.
+template <int EPI>
+hipError_t launch_vt_gemm(const float* a, int64_t lda, int64_t a_rows, const float* w, int64_t M,
+                          int64_t K, int64_t N, const VtEpi& ep, hipStream_t st) {
+    if (M <= 0 || N <= 0) return hipSuccess;
+    constexpr bool DIST = EPI == kEpiDist;
+    auto tiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+    const double us = DIST ? 7.0 + (double)((tiles(64, 128) + 255) / 256) *
+                                       (1.05 * (double)((K + 31) / 32) + 0.8)
+                           : f32_small_us(M, N, K);
+    int tile = -1;
+    if (K > 0 && slice_best_tile_f32(M, N, K, false, &tile) < us)
+        return launch_vt_slice<EPI>(tile, a, lda, a_rows, w, M, K, N, ep, st);
+    if constexpr (DIST) {
+        if (tiles(128, 128) > kVtLargeTiles)
+            return launch_vt_tile<VtLarge, EPI>(a, lda, a_rows, w, M, K, N, ep, st);
+        return launch_vt_tile<VtWide, EPI>(a, lda, a_rows, w, M, K, N, ep, st);
+    } else {
+        return launch_vt_tile<VtSmall, EPI>(a, lda, a_rows, w, M, K, N, ep, st);
+    }
 }
 
 __device__ __forceinline__ float block_sum256(float v, float* red) {

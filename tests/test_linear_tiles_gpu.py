@@ -79,3 +79,19 @@ def test_tile_fused_epilogues(ncm, oracle, cuda, m, k, inter, bias):
     kernels.rope_rotate(ref[:, :rot], rot // 64, 64, seq, cd, sd)
     got = kernels.linear_bf16_rope64(x, w, rot, seq, cd, sd, bias=b)
     assert torch.equal(got.view(torch.int16), ref.view(torch.int16))
+
+
+# fp32: the 64x64 tiles at ragged M, N and K, and 128x128 in six rounds.
+@pytest.mark.parametrize("m,k,n", [(700, 100, 8190), (333, 36, 30003), (500, 576, 49100)])
+def test_f32_tiles(ncm, cuda, m, k, n):
+    import torch
+    from ncmorph_amd import kernels
+
+    print(f"f32 tile m={m} k={k} n={n}", flush=True)
+    g = torch.Generator(device=cuda).manual_seed(m + k + n)
+    x = torch.randn(m, k, generator=g, device=cuda)
+    w = torch.randn(n, k, generator=g, device=cuda)
+    y = kernels.linear_f32(x, w)
+    ref = x.double() @ w.double().t()
+    bound = (x.double().abs() @ w.double().abs().t()) * (k + 1) * 2.0**-24
+    assert bool(((y.double() - ref).abs() <= bound).all())
