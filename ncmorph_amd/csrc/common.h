@@ -67,9 +67,9 @@ __device__ __forceinline__ void add_flush16(f32x16_t& v, float b) {
 }
 
 // g / (1 + exp(-g)), to be rounded to bf16: exp(-g) as exp2 of -g times the
-// upper 16 bits of log2 e (exact in fp32 for a bf16 g, which has 8 bits), corrected to first order for the rest, and v_rcp_f32 for the
-// division; about 2 fp32 ulps in all, at a third of expf and the IEEE
-// division's instructions. Over all 65,280 finite g the bf16 result is that of
+// upper 16 bits of log2 e (exact in fp32 for a bf16 g, which has 8 bits),
+// corrected to first order for the rest, and v_rcp_f32 for the division; about
+// 2 fp32 ulps in all, at a third of expf and the IEEE division's instructions. Over all 65,280 finite g the bf16 result is that of
 // the exact quotient but for at most two within 2 ulps of a rounding boundary.
 // Past |g| = 150 the exponential has saturated (the clamp keeps its correction
 // from being infinity times zero).
