@@ -288,11 +288,20 @@ hipError_t launch_slice(int tile, const SliceArgs& a, hipStream_t st) {
 // tile covers M, every weight is read once and the weight stream is the
 // bound at any N: 64 rows, 128256 x 2048 162 -> 139 us, 28672 x 4096 55.9 ->
 // 54.8 us; from 65 rows on a wide N would be read twice (77 rows, 28672 x 4096:
-// 54 -> 61 us).
+// 54 -> 61 us). The largest tile sums eight wavefronts' 20 blocks after a K loop
+// that, up to K = 640, is shorter than that, and with one row tile of 65 to 80 rows
+// up to 1024: the 64 x 128 tiles take those (77 rows, 9728 x 576 / x 896: 9.6 -> 8.1 /
+// 11.6 -> 10.2 us; 150 rows, 6144 x 576 9.0 -> 8.1; 1100 rows, 1152 x 576 8.4 -> 7.5; but
+// 300 rows, 4096 x 1024 10.5 -> 11.4, 77 rows, 14336 x 4096 31.8 -> 33.9).
+constexpr int64_t kLargestTile = 9;  // cost of a round of the 5 x 4 tile
+
 bool linear_slice_fits(int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || N <= 0 || K <= 0 || K > (int64_t)1 << 21) return false;
+    if (M <= 64) return true;
     int tile;
-    return M <= 64 || best_tile(M, N, false, &tile) <= 13;
+    const int64_t cost = best_tile(M, N, false, &tile);
+    if (cost == kLargestTile && (K <= 640 || (K <= 1024 && M <= 80))) return false;
+    return cost <= 13;
 }
 
 hipError_t launch_linear_slice(const uint16_t* x, const uint16_t* w, const uint16_t* bias,

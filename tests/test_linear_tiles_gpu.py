@@ -23,7 +23,7 @@ def _dev(rng, shape, std, cuda):
 
 # 64x128 (one round, two row tiles and six), 128x256 (one row tile, three, two
 # rounds), 128x128 (one round and three), 256x256.
-@pytest.mark.parametrize("m,k,n", [(128, 136, 16383), (350, 72, 5000), (128, 64, 49153),
+@pytest.mark.parametrize("m,k,n", [(128, 136, 16383), (350, 72, 5000), (77, 520, 9999), (128, 64, 49153),
                                    (300, 328, 40001), (1100, 8, 14000), (1500, 72, 2049), (600, 72, 15900),
                                    (600, 520, 9000), (2047, 200, 8190)])
 def test_tile_outputs(ncm, cuda, m, k, n):
