@@ -363,7 +363,7 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const float* __restrict__
         return;
     }
     auto act = [](float v, float u) {
-        const float a = __uint_as_float(bf16_bits_rne(silu_near<false>(v)) << 16);
+        const float a = __uint_as_float(bf16_bits_rne(v / (1.0f + expf(-v))) << 16);
         return bf16_bits_rne(a * u);
     };
     const int64_t i0 = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
@@ -378,7 +378,8 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const float* __restrict__
         // the NaN rule on the stored one (a NaN stays a NaN through a * u).
 #pragma unroll
         for (int e = 0; e < 4; e += 2) {
-            const uint32_t a = bf16x2_rne(silu_near<false>(g[e]), silu_near<false>(g[e + 1]));
+            const uint32_t a = bf16x2_rne(g[e] / (1.0f + expf(-g[e])),
+                                          g[e + 1] / (1.0f + expf(-g[e + 1])));
             const uint32_t r = bf16x2_bits_rne(__uint_as_float(a << 16) * u[e],
                                                __uint_as_float(a & 0xFFFF0000u) * u[e + 1]);
             b[e] = r & 0xFFFFu;
