@@ -3,6 +3,8 @@
 #include "common.h"
 #include "rvq.h"
 
+#include <type_traits>
+
 namespace ncm {
 
 static bool pow2(int64_t s) { return s >= 1 && (s & (s - 1)) == 0; }
@@ -73,122 +75,137 @@ hipError_t launch_rvq_csq(const uint16_t* codebooks, int64_t rows, int64_t d, fl
 }
 
 // recon[b, t, :] = sum over l (in order, from +0) of C_l[code_l[b, t / s_l]].
-// A wavefront takes R consecutive rows (so every code is one scalar load) and
-// 64 VEC of their columns, VEC to a lane, and issues the code rows of eight
-// levels together. R = 4 (t a multiple of 4, so the rows share a sequence and
-// every code of stride 4 or more): such a level's row is loaded once for the
-// four, a stride-2 level's twice. Consecutive rows stay on one XCD, whose L2
-// then holds the coarse levels' rows that they share. Bound: writing recon and
-// reading the finest levels' code rows (402 MB at 16 x 2048 x 2048, 8 levels).
-// There: 283 us with one thread per four columns of a row and 64-bit divisions
-// for every level's position (VALU), 172 us with R = 1, 131 us with R = 4.
-template <int VEC, int R>
-__global__ __launch_bounds__(256) void rvq_decode_kernel(const int32_t* __restrict__ codes,
-                                                         uint32_t t, int64_t d, LevelTable L,
-                                                         const uint16_t* __restrict__ cb,
-                                                         int64_t v, float* __restrict__ recon,
-                                                         uint32_t rows) {
-    constexpr int W = VEC / 2;  // 32-bit words of VEC bf16 values
-    typedef uint32_t words_t __attribute__((ext_vector_type(W)));
-    const uint32_t group = (uint32_t)xcd_remap((int)blockIdx.x, (int)gridDim.x);
-    const uint32_t row = __builtin_amdgcn_readfirstlane((group * 4 + (threadIdx.x >> 6)) * R);
-    if (row >= rows) return;
-    const int64_t col = ((int64_t)blockIdx.y * 64 + (threadIdx.x & 63)) * VEC;
-    if (col >= d) return;
+// A thread takes eight columns of R consecutive rows; a workgroup takes
+// `chunks` such pieces of each of `groups` row groups, as many as fill its
+// wavefronts. The codes of up to eight code rows are loaded together, then
+// those rows, then they are added in level order; R = 4 (t a multiple of 4, so
+// the rows share a sequence and every code of stride 4 or more) loads a level
+// below n4 once for its four rows and one below n2 twice. Consecutive rows
+// stay on one XCD, whose L2 then holds the coarse levels' rows that they share.
+//
+// Bound: writing recon and reading the finest levels' code rows. Against one
+// thread per four columns, with 64-bit divisions for every level's position, us
+// (1024 codes): 32768 rows of d 2048, strides 128 .. 1 217 -> 79, four levels of
+// stride 1 131 -> 66, one level 55 -> 55; of d 576, four of stride 1 40 -> 22; 262144
+// rows of d 64, strides 128 .. 1 55 -> 19, four of stride 1 33 -> 19, one 16.8 -> 15.8.
+// (A wavefront per row or four rows, with its lanes past d idle and its loads
+// always those of eight levels: 98, 104, 84, 55, 82, 109 and 103.)
+template <int R>
+__global__ __launch_bounds__(512) void rvq_decode_kernel(
+    const int32_t* __restrict__ codes, uint32_t t, int64_t d, LevelTable L,
+    const uint16_t* __restrict__ cb, int64_t v, float* __restrict__ recon, uint32_t rows,
+    uint32_t chunks, uint32_t groups, int n4, int n2) {
+    const uint32_t block = (uint32_t)xcd_remap((int)blockIdx.x, (int)gridDim.x);
+    const uint32_t g = threadIdx.x / chunks, c = threadIdx.x - g * chunks;
+    const uint64_t first = ((uint64_t)block * groups + g) * R;
+    const int64_t col = ((int64_t)blockIdx.y * chunks + c) * 8;
+    if (g >= groups || first >= rows || col >= d) return;
+    const uint32_t row = (uint32_t)first;
     const uint32_t bb = row / t, tt = row - bb * t;
     const int32_t* cr = codes + bb * L.total;
-    float a[R][VEC];
+    float a[R][8];
 #pragma unroll
     for (int r = 0; r < R; ++r)
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) a[r][e] = 0.0f;
-    auto code_row = [&](int l, uint32_t pos) {
-        int32_t k = cr[L.offset[l] + pos];
-        k = k < 0 ? 0 : (k >= v ? (int32_t)(v - 1) : k);
-        return *(const words_t*)(cb + ((int64_t)l * v + k) * d + col);
-    };
-    auto add = [&](int r, const words_t& p) {
+        for (int e = 0; e < 8; ++e) a[r][e] = 0.0f;
+    // N levels from l on, S code rows each (every R / S rows share one).
+    auto batch = [&](auto n, auto s, int l) {
+        constexpr int N = decltype(n)::value, S = decltype(s)::value;
+        int32_t k[N][S];
 #pragma unroll
-        for (int e = 0; e < W; ++e) {
-            a[r][2 * e] = a[r][2 * e] + bf16_lo_to_f32(p[e]);
-            a[r][2 * e + 1] = a[r][2 * e + 1] + bf16_hi_to_f32(p[e]);
-        }
-    };
-    for (int l0 = 0; l0 < L.levels; l0 += 8) {
-        words_t p[8][R];
+        for (int i = 0; i < N; ++i)
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            // Past the last level: its row again, not added.
-            const int l = l0 + i < L.levels ? l0 + i : L.levels - 1;
-            const int sh = __builtin_ctz((uint32_t)L.stride[l]);
-            p[i][0] = code_row(l, tt >> sh);
-            if constexpr (R == 4) {
-                if (sh < 2) p[i][2] = code_row(l, (tt + 2) >> sh);
-                if (sh < 1) {
-                    p[i][1] = code_row(l, tt + 1);
-                    p[i][3] = code_row(l, tt + 3);
-                }
+            for (int j = 0; j < S; ++j)
+                k[i][j] = cr[L.offset[l + i] +
+                             ((tt + j * (R / S)) >> __builtin_ctz((uint32_t)L.stride[l + i]))];
+        u32x4_t p[N][S];
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+#pragma unroll
+            for (int j = 0; j < S; ++j) {
+                const int32_t kk = k[i][j] < 0 ? 0 : (k[i][j] >= v ? (int32_t)(v - 1) : k[i][j]);
+                p[i][j] = *(const u32x4_t*)(cb + ((int64_t)(l + i) * v + kk) * d + col);
             }
-        }
         // Every load in flight before the first sum (the compiler would fold
         // each row as it comes to save registers).
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            if (l0 + i >= L.levels) break;
-            add(0, p[i][0]);
-            if constexpr (R == 4) {
-                const int stride = L.stride[l0 + i];
-                if (stride == 1) {
-                    add(1, p[i][1]);
-                    add(2, p[i][2]);
-                    add(3, p[i][3]);
-                } else {
-                    add(1, p[i][0]);
-                    if (stride == 2) {
-                        add(2, p[i][2]);
-                        add(3, p[i][2]);
-                    } else {
-                        add(2, p[i][0]);
-                        add(3, p[i][0]);
-                    }
+        for (int i = 0; i < N; ++i)
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const uint32_t w = p[i][r / (R / S)][e];
+                    a[r][2 * e] = a[r][2 * e] + bf16_lo_to_f32(w);
+                    a[r][2 * e + 1] = a[r][2 * e + 1] + bf16_hi_to_f32(w);
                 }
+    };
+    // Levels [l, end): eight code rows at a time, then what is left by halves.
+    auto levels = [&](auto s, int l, int end) {
+        constexpr int S = decltype(s)::value;
+        for (; l + 8 / S <= end; l += 8 / S) batch(std::integral_constant<int, 8 / S>{}, s, l);
+        if constexpr (S < 2)
+            if (l + 4 <= end) {
+                batch(std::integral_constant<int, 4>{}, s, l);
+                l += 4;
             }
-        }
+        if constexpr (S < 4)
+            if (l + 2 <= end) {
+                batch(std::integral_constant<int, 2>{}, s, l);
+                l += 2;
+            }
+        if (l < end) batch(std::integral_constant<int, 1>{}, s, l);
+    };
+    if constexpr (R == 4) {
+        levels(std::integral_constant<int, 1>{}, 0, n4);
+        levels(std::integral_constant<int, 2>{}, n4, n2);
+        levels(std::integral_constant<int, 4>{}, n2, L.levels);
+    } else {
+        levels(std::integral_constant<int, 1>{}, 0, L.levels);
     }
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         float* o = recon + (int64_t)(row + r) * d + col;
-#pragma unroll
-        for (int e = 0; e < VEC; e += 4)
-            *(f32x4_t*)(o + e) = f32x4_t{a[r][e], a[r][e + 1], a[r][e + 2], a[r][e + 3]};
+        *(f32x4_t*)o = f32x4_t{a[r][0], a[r][1], a[r][2], a[r][3]};
+        *(f32x4_t*)(o + 4) = f32x4_t{a[r][4], a[r][5], a[r][6], a[r][7]};
     }
 }
 
-constexpr int64_t kDecodeFourRows = 4096;
+// Elements of recon from which a thread takes four rows: an output of 256 MB,
+// which the memory-side cache does not hold (one row -> four: 32768 x 2048, strides
+// 128 .. 1 96 -> 79 us; 262144 x 512, one level 149 -> 103). Below, four rows leave too
+// few loads in flight (32768 x 1024, one level 25.9 -> 28.9).
+constexpr int64_t kDecodeFourRows = (int64_t)1 << 26;
 
 hipError_t launch_rvq_decode(const int32_t* codes, int64_t b, int64_t t, int64_t d,
                              int64_t levels, const int32_t* strides, const uint16_t* codebooks,
                              int64_t v, float* recon, hipStream_t stream) {
     const LevelTable L = make_level_table(t, levels, strides);
     const int64_t rows = b * t;  // at most 2^31; strides are powers of two, d % 64 == 0
-    // Four rows a wavefront where there are enough of them to fill the chip.
-    // Narrow rows: four columns to a lane fill the wavefront.
-    const bool four = t % 4 == 0 && rows >= kDecodeFourRows;
-    const int64_t per = four ? 16 : 4;
-    const unsigned gx = (unsigned)((rows + per - 1) / per);
-#define NCM_DEC(VEC, R)                                                                          \
-    hipLaunchKernelGGL((rvq_decode_kernel<VEC, R>),                                              \
-                       dim3(gx, (unsigned)((d + 64 * VEC - 1) / (64 * VEC))), dim3(256), 0,      \
-                       stream, codes, (uint32_t)t, d, L, codebooks, v, recon, (uint32_t)rows)
-    if (d >= 512) {
-        if (four) NCM_DEC(8, 4);
-        else NCM_DEC(8, 1);
-    } else {
-        if (four) NCM_DEC(4, 4);
-        else NCM_DEC(4, 1);
+    int n4 = 0, n2 = 0;          // strides do not increase
+    for (int l = 0; l < L.levels; ++l) {
+        n4 += L.stride[l] >= 4;
+        n2 += L.stride[l] >= 2;
     }
-#undef NCM_DEC
+    const bool four = t % 4 == 0 && rows * d >= kDecodeFourRows;
+    // 256 columns at a time, so that an XCD's L2 holds more of the codebooks' rows
+    // (32768 x 2048, 1024 codes, four full-resolution levels 102 -> 66 us); four rows
+    // and at most one such level read fewer rows than they write and take whole rows up to 4096
+    // columns (strides 128 .. 1, 83 -> 79; with 4096 codes 112 -> 98).
+    const int64_t most = four && L.levels - n2 < 2 ? 512 : 32;
+    const int64_t shares = (d / 8 + most - 1) / most, chunks = (d / 8 + shares - 1) / shares;
+    // Of the workgroup sizes the one that whole row pieces fill best.
+    int64_t threads = (chunks + 63) / 64 * 64, groups = threads / chunks;
+    for (int64_t n = threads + 64; n <= 512; n += 64)
+        if (n / chunks * threads > groups * n) {
+            threads = n;
+            groups = n / chunks;
+        }
+    const int64_t per = groups * (four ? 4 : 1);
+    const dim3 grid((unsigned)((rows + per - 1) / per), (unsigned)shares);
+    hipLaunchKernelGGL(four ? rvq_decode_kernel<4> : rvq_decode_kernel<1>, grid,
+                       dim3((unsigned)threads), 0, stream, codes, (uint32_t)t, d, L, codebooks, v,
+                       recon, (uint32_t)rows, (uint32_t)chunks, (uint32_t)groups, n4, n2);
     return hipGetLastError();
 }
 

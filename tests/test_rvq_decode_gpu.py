@@ -1,6 +1,7 @@
-"""RVQ decode where its wavefronts change shape: four rows each (t a multiple of
-4, 4096 rows or more) and one, rows narrower and wider than 512, strides of 1,
-2, 4 and more, and more than eight levels: bit-identical to the oracle."""
+"""RVQ decode where its workgroups change shape: one row a thread and four (t a
+multiple of 4, 2^26 elements or more), widths whose pieces fill the wavefronts
+or leave lanes over, in one share or several, strides of 1, 2, 4 and more, and
+level counts that leave every remainder of eight: bit-identical to the oracle."""
 import numpy as np
 import pytest
 
@@ -16,6 +17,13 @@ pytestmark = pytest.mark.gpu
     (4, 1024, 512, (16, 8, 8, 4, 4, 2, 2, 1, 1), 33),
     (3, 1366, 128, (2, 1), 20),
     (1, 8, 2048, (8, 1), 5),
+    (1, 33, 192, (1,) * 7, 9),
+    (1, 37, 4160, (1,) * 3, 9),
+    (2, 40, 1088, (8, 4, 4, 4, 4, 4), 9),
+    # 2^26 elements and more: four rows a thread; the third one row (t odd).
+    (4, 4100, 4096, (4, 2, 1), 12),
+    (2, 16392, 2112, (8, 8, 4, 2, 2, 2, 1, 1, 1), 12),
+    (1, 16387, 4096, (1, 1), 12),
 ])
 def test_decode_shapes(ncm, oracle, cuda, b, t, d, strides, v):
     import torch
@@ -30,6 +38,22 @@ def test_decode_shapes(ncm, oracle, cuda, b, t, d, strides, v):
                     torch.from_numpy(cb.view(np.int16)).to(cuda).view(torch.bfloat16), strides, t)
     want = oracle.rvq_decode(np.clip(codes, 0, v - 1), cb, strides, t)
     assert np.array_equal(got.cpu().numpy().view(np.uint32), want.view(np.uint32))
+
+
+def test_decode_of_many_narrow_rows(ncm, cuda):
+    """More than 2^26 rows of 64 columns: the grid has 8 threads a row, of at
+    most 2^32."""
+    import torch
+    from ncmorph_amd import vq
+
+    t = 2**26 + 2
+    cb = torch.arange(3 * 64, dtype=torch.float32, device=cuda).reshape(1, 3, 64)
+    cb = cb.to(torch.bfloat16)
+    codes = (torch.arange(t, dtype=torch.int32, device=cuda) * 7 % 3).reshape(1, t)
+    got = vq.decode(codes, cb, (1,), t)
+    for r0 in range(0, t, 2**24):
+        want = cb[0].float()[codes[0, r0:r0 + 2**24].long()]
+        assert torch.equal(got[0, r0:r0 + 2**24], want), r0
 
 
 @pytest.mark.parametrize("b,t,d,levels,v", [(1, 1, 64, 1, 1), (1, 128, 256, 4, 512),
