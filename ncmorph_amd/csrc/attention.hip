@@ -844,7 +844,14 @@ hipError_t launch_attn_hd(const uint16_t* q, const uint16_t* k, const uint16_t* 
                           int64_t kv_stride, int64_t out_stride, int64_t window, SegArgs sa,
                           int out_mode, uint16_t* vt, hipStream_t stream) {
     constexpr int NWV = attn_waves<HD>();
-    if (MASK == 0 && T <= kShortKeys && (T + 31) / 32 * hq * batch <= short_groups<HD>())
+    // The V^T copy lets `out` lie over v (the kernels after it read the copy);
+    // the short kernel reads v while other workgroups already store.
+    const uintptr_t v0 = (uintptr_t)v, o0 = (uintptr_t)out;
+    const uintptr_t v1 = v0 + 2 * (uint64_t)((batch * T - 1) * kv_stride + hkv * HD);
+    const uintptr_t o1 = o0 + (out_mode == NCM_OUT_BF16 ? 2 : 4) *
+                                  (uint64_t)((batch * T - 1) * out_stride + hq * HD);
+    if (MASK == 0 && T <= kShortKeys && (T + 31) / 32 * hq * batch <= short_groups<HD>() &&
+        (o1 <= v0 || v1 <= o0))
         return launch_attn_short<HD>(q, k, v, out, batch, T, hq, hkv, q_stride, kv_stride,
                                      out_stride, window, out_mode, stream);
     const int64_t Tp = attention_vt_padded(T);

@@ -1372,8 +1372,10 @@ int rvq_encode_ws(hipStream_t st, void* ws, size_t ws_bytes, const float* x, int
 
     hipError_t e = hipSuccess;
     if (flat_fits(b * t, d, v, strides, gap != nullptr, n_flagged || counts)) {
-        const FlatArgs fa{x, codebooks, csq, force_codes, codes, recon, t, d, v, b * t,
-                          (int)levels};
+        // Forced codes in `codes` itself are each row's own by the time they are read
+        // (one wavefront writes and reads them in rvq_rescore_kernel); here eight would race.
+        const FlatArgs fa{x, codebooks, csq, force_codes == codes ? nullptr : force_codes, codes,
+                          recon, t, d, v, b * t, (int)levels};
         const dim3 grid((unsigned)(b * t)), block(64 * kFlatWaves);
         if (d <= 256)
             hipLaunchKernelGGL(rvq_flat_kernel<1>, grid, block, 0, st, fa);

@@ -40,3 +40,29 @@ def test_short_causal_attention(ncm, oracle, cuda, hd, t, window):
         err = np.abs(out[rows] - ref)
         assert np.all(err <= 2.0**-7 * np.abs(ref) + 2.0**-7 * np.max(np.abs(vf[rows]))), b
         assert np.mean(out[rows] == ref) >= 0.99, np.mean(out[rows] == ref)
+
+
+@pytest.mark.parametrize("hd,t", [(64, 77), (64, 256), (128, 130)])
+def test_short_output_over_v(ncm, cuda, hd, t):
+    """`out` may be v itself: every element of v is read before it is
+    overwritten. Within the two kernels' difference (one rounding of a
+    probability at 2^-8) of the same call with an output of its own."""
+    import torch
+    from ncmorph_amd import kernels
+
+    g = torch.Generator(device=cuda).manual_seed(hd + t)
+    batch, heads = 3, 4
+    q, k, v = (torch.randn(batch * t, heads * hd, generator=g, device=cuda).to(torch.bfloat16)
+               for _ in range(3))
+    want = kernels.attention_bf16(q, k, v, batch, t, heads, heads, hd, out_mode="bf16")
+    want, peak = want.float(), float(v.float().abs().max())
+    for _ in range(3):
+        w = v.clone()
+        got = kernels.attention_bf16(q, k, w, batch, t, heads, heads, hd, out_mode="bf16", out=w)
+        assert float((got.float() - want).abs().max()) <= 2.0**-7 * peak
+    # Beside v in one buffer of rows.
+    qkv = torch.cat([q, k, v], 1)
+    cols = [slice(i * heads * hd, (i + 1) * heads * hd) for i in range(3)]
+    got = kernels.attention_bf16(qkv[:, cols[0]], qkv[:, cols[1]], qkv[:, cols[2]], batch, t, heads,
+                                 heads, hd, out_mode="bf16", out=qkv[:, cols[2]])
+    assert float((got.float() - want).abs().max()) <= 2.0**-7 * peak

@@ -85,6 +85,24 @@ def test_full_resolution_encode(ncm, oracle, cuda, b, t, d, levels, v):
                           forced["recon"].view(np.uint32))
 
 
+@pytest.mark.parametrize("want_gap", [False, True])
+def test_forced_codes_in_the_output(ncm, cuda, want_gap):
+    """force_codes may be the codes output: every code is the library's own by
+    the time it is read, so the encode is the unforced one, in the one launch
+    of few rows as in the general path."""
+    import torch
+    from ncmorph_amd import vq
+
+    x, cb = synth.rvq_inputs(3, 1, 100, 192, 4, 500)
+    xd = torch.from_numpy(x).to(cuda)
+    cbd = torch.from_numpy(cb.view(np.int16)).to(cuda).view(torch.bfloat16)
+    own = vq.encode(xd, cbd, (1,) * 4, want_gap=want_gap)
+    for _ in range(3):
+        buf = torch.zeros((1, 400), dtype=torch.int32, device=cuda)
+        r = vq.encode(xd, cbd, (1,) * 4, want_gap=want_gap, force_codes=buf, out={"codes": buf})
+        assert torch.equal(r["codes"], own["codes"]) and torch.equal(r["recon"], own["recon"])
+
+
 @pytest.mark.parametrize("d,v", [(64, 65), (320, 300)])
 def test_full_resolution_rows_without_a_distance(ncm, oracle, cuda, d, v):
     """Rows that hold NaN or infinities get the codes of the general path,
