@@ -14,12 +14,12 @@ namespace ncm {
 // vector sum, lanes into the scalar sum) run in the reference's order on
 // values gathered by shuffles. Every product and sum is a separate fp32 op
 // (built with -ffp-contract=off), as in the reference.
-// Widths 1024, 2048 and 4096 (the decoder and NCM hidden sizes) hold the
-// row in registers for both passes (rms_norm_rows_reg_kernel: 8224 x 4096
-// rows measured 53.5 -> 39.0 us, 4096 x 2048 11.95 -> 10.7 us). Other widths
-// read the row from global memory twice (the second pass mostly from the
-// caches): staging it in LDS measured slower at widths 2048-8192, since the
-// 16 KB-per-row stages held the kernel to two workgroups per CU.
+// Widths that are multiples of 32, kRmsRegMin to kRmsRegMax, hold the row in registers
+// for both passes (rms_norm_rows_reg_kernel: 8224 x 4096 rows measured 53.5 ->
+// 39.0 us, 4096 x 2048 11.95 -> 10.7 us). Other widths read the row from global
+// memory twice (the second pass mostly from the caches): staging it in LDS
+// measured slower at widths 2048-8192, since the 16 KB-per-row stages held the
+// kernel to two workgroups per CU.
 
 // The pinned sum of squares of one row (root.zig:152-227) by one
 // wavefront: lane c < 32 runs chain (r = c / 8, l = c % 8) with its four
@@ -176,13 +176,15 @@ __device__ __forceinline__ void rms_write_row(const float* __restrict__ x,
     }
 }
 
-// Widths 64 NR: one row per
-// wavefront, read once and held in registers (lane j holds x[64 i + j] in
-// v[i]) for both passes, instead of the second pass reading the row again.
-// The pinned cascade above, on the same chains: chain c = lane c < 32 takes
-// x[32 q + c] as its q-th element, which is v[q / 2] of lane c for even q
-// and of lane c + 32 for odd q (a permlane32 swap), in the same order with
-// the same operations, so the sum has the same bits.
+// 64 LOW < n <= 64 NR elements, a multiple of 32: one row per wavefront, read once and
+// held in registers (lane j holds x[64 i + j] in v[i], zero past the row) for
+// both passes, instead of the second pass reading the row again. The pinned
+// cascade above, on the same chains: chain c = lane c < 32 takes x[32 q + c] as
+// its q-th element, which is v[q / 2] of lane c for even q and of lane c + 32
+// for odd q (a permlane32 swap), in the same order with the same operations,
+// so the sum has the same bits. The zeros past the row change none: they add
+// +0 to sums of squares, and a last run that they complete is added to the
+// level above it as the cascade's end would add it.
 constexpr int rms_ilog2_ceil(int v) {
     int lg = 0;
     while ((1 << lg) < v) ++lg;
@@ -192,6 +194,7 @@ constexpr int rms_ilog2_ceil(int v) {
 template <int NR>
 __device__ __forceinline__ float rms_sum_squares_reg(const float (&v)[NR], int lane) {
     constexpr int groups = 2 * NR;
+    static_assert(groups < 256, "one level above the runs");
     constexpr int lg = rms_ilog2_ceil(groups);
     constexpr int power = lg / 4 > 4 ? lg / 4 : 4;
     constexpr int step = 1 << power, mask = step - 1;
@@ -244,35 +247,56 @@ __device__ __forceinline__ float rms_sum_squares_reg(const float (&v)[NR], int l
     return sum;
 }
 
-template <int OUT_MODE, int NR, bool FEW>
+template <int OUT_MODE, int LOW, int NR, bool FEW>
 __global__ __launch_bounds__(256) void rms_norm_rows_reg_kernel(const float* __restrict__ x,
                                                                 const float* __restrict__ weight,
                                                                 void* __restrict__ y,
-                                                                int64_t rows, float epsilon) {
-    constexpr int64_t n = 64 * NR;
+                                                                int64_t rows, int n,
+                                                                float epsilon) {
     const int lane = threadIdx.x & 63;
     const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= rows) return;
-    // Buffer loads: the row's base in the resource, the lane's offset in one
-    // VGPR, each 256-byte step in the scalar offset.
+    // Buffer accesses: the row in the resource, so that past it loads give zero
+    // and stores do nothing (where neither can happen, stores are plain); the
+    // lane's offset in one VGPR, each load's step in the scalar offset, or where
+    // it may pass the row in the offset that is checked.
+    constexpr int kOut = OUT_MODE == NCM_OUT_BF16 ? 2 : 4;
     const __amdgpu_buffer_rsrc_t rx = make_rsrc(x + row * n, (uint32_t)(n * 4));
     const __amdgpu_buffer_rsrc_t rw = make_rsrc(weight, (uint32_t)(n * 4));
-    const uint32_t lo = 4u * (uint32_t)lane;
+    const __amdgpu_buffer_rsrc_t ry = make_rsrc((char*)y + row * n * kOut, (uint32_t)(n * kOut));
+    const uint32_t lo = 4u * (uint32_t)lane, so = (uint32_t)(kOut * lane);
+    auto load = [&](__amdgpu_buffer_rsrc_t r, int i) {
+        return __uint_as_float(
+            i < LOW ? __builtin_amdgcn_raw_buffer_load_b32(r, lo, 256 * i, 0)
+                    : __builtin_amdgcn_raw_buffer_load_b32(r, lo + 256 * i, 0, 0));
+    };
+    auto store = [&](int i, uint32_t bits) {
+        const int64_t e = row * n + 64 * i + lane;
+        if constexpr (OUT_MODE == NCM_OUT_BF16) {
+            if (i < LOW)
+                ((uint16_t*)y)[e] = (uint16_t)bits;
+            else
+                __builtin_amdgcn_raw_buffer_store_b16((uint16_t)bits, ry, so + 128 * i, 0, 0);
+        } else {
+            if (i < LOW)
+                ((uint32_t*)y)[e] = bits;
+            else
+                __builtin_amdgcn_raw_buffer_store_b32(bits, ry, so + 256 * i, 0, 0);
+        }
+    };
     float v[NR];
 #pragma unroll
-    for (int i = 0; i < NR; ++i)
-        v[i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rx, lo, 256 * i, 0));
+    for (int i = 0; i < NR; ++i) v[i] = load(rx, i);
     // FEW: the weight's loads fly during the sum (twice the registers, which
     // cost occupancy and time when there are many rows).
     float wr[FEW ? NR : 1];
     if constexpr (FEW) {
 #pragma unroll
-        for (int i = 0; i < NR; ++i)
-            wr[i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rw, lo, 256 * i, 0));
+        for (int i = 0; i < NR; ++i) wr[i] = load(rw, i);
     }
     auto weight_at = [&](int i) {
         if constexpr (FEW) return wr[i];
-        return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rw, lo, 256 * i, 0));
+        return load(rw, i);
     };
     const float sum = rms_sum_squares_reg<NR>(v, lane);
     const float mean = sum / (float)n;
@@ -282,29 +306,20 @@ __global__ __launch_bounds__(256) void rms_norm_rows_reg_kernel(const float* __r
 #pragma unroll
     for (int i = 0; i < NR; i += 2) {
         if (!FEW && i % 8 == 0) __builtin_amdgcn_sched_barrier(0);
-        // An odd NR's last pair has one element.
-        const bool two = i + 1 < NR;
-        const float w0 = weight_at(i), w1 = two ? weight_at(two ? i + 1 : i) : 0.0f;
-        const float v1 = two ? v[two ? i + 1 : i] : 0.0f;
-        const int64_t e0 = row * n + 64 * i + lane, e1 = e0 + 64;
+        const float w0 = weight_at(i), w1 = weight_at(i + 1);
         if (OUT_MODE == NCM_OUT_F32) {
-            const float n0 = v[i] * inv, n1 = v1 * inv;
-            ((float*)y)[e0] = n0 * w0;
-            if (two) ((float*)y)[e1] = n1 * w1;
+            const float n0 = v[i] * inv, n1 = v[i + 1] * inv;
+            store(i, __float_as_uint(n0 * w0));
+            store(i + 1, __float_as_uint(n1 * w1));
             continue;
         }
-        const uint32_t nb = bf16x2_rne(v[i] * inv, v1 * inv);
+        const uint32_t nb = bf16x2_rne(v[i] * inv, v[i + 1] * inv);
         const uint32_t wb = bf16x2_rne(w0, w1);
         const uint32_t r = bf16x2_bits_rne(
             __uint_as_float(nb << 16) * __uint_as_float(wb << 16),
             __uint_as_float(nb & 0xFFFF0000u) * __uint_as_float(wb & 0xFFFF0000u));
-        if (OUT_MODE == NCM_OUT_BF16) {
-            ((uint16_t*)y)[e0] = (uint16_t)(r & 0xFFFFu);
-            if (two) ((uint16_t*)y)[e1] = (uint16_t)(r >> 16);
-        } else {
-            ((float*)y)[e0] = __uint_as_float(r << 16);
-            if (two) ((float*)y)[e1] = __uint_as_float(r & 0xFFFF0000u);
-        }
+        store(i, OUT_MODE == NCM_OUT_BF16 ? r & 0xFFFFu : r << 16);
+        store(i + 1, OUT_MODE == NCM_OUT_BF16 ? r >> 16 : r & 0xFFFF0000u);
     }
 }
 
@@ -613,37 +628,50 @@ hipError_t launch_bias_round(void* y, const float* bias, int64_t rows, int64_t n
 
 // Rows up to which the register kernel's wavefronts run one or two to a SIMD:
 // its time is then the latency of one wavefront, and it loads the weight up
-// front (77 x 2048 in bf16: 4.8 -> 4.2 us; 200 x 576 in fp32, which the two-pass
-// kernel took before: 6.4 -> 3.1 us).
+// front (77 x 2048 in bf16: 4.8 -> 4.2 us; 200 x 576 in fp32, two-pass kernel 6.4 ->
+// 3.1 us).
 constexpr int64_t kRmsFewRows = 2048;
+// Widths of the register kernel: above kRmsRegMin (at 64 the two-pass kernel's
+// two rows a wavefront are faster from 16384 rows on: 56.7 us against 67.6 for
+// 400000; at 128 146 -> 106) and up to kRmsRegMax, the widest whose weights fit the
+// registers too (5120: 200 rows 18.6 -> 6.5 us, 4096 rows 43 -> 28).
+constexpr int64_t kRmsRegMin = 64, kRmsRegMax = 5120;
 
 template <int OUT_MODE>
 static hipError_t launch_rms_t(const float* x, const float* weight, void* y, int64_t rows,
                                int64_t n, float epsilon, hipStream_t stream) {
-    // The register kernel for the widths it is built for: the hidden sizes of
-    // the checkpoints whose configurations the tests hold.
-    const bool few = rows <= kRmsFewRows;
-#define NCM_RMS(NR)                                                                          \
-    case 64 * NR:                                                                            \
-        if (few)                                                                             \
-            hipLaunchKernelGGL((rms_norm_rows_reg_kernel<OUT_MODE, NR, true>),               \
-                               dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream, x,    \
-                               weight, y, rows, epsilon);                                    \
-        else                                                                                 \
-            hipLaunchKernelGGL((rms_norm_rows_reg_kernel<OUT_MODE, NR, false>),              \
-                               dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream, x,    \
-                               weight, y, rows, epsilon);                                    \
-        return hipGetLastError();
-    switch (n) {
-        NCM_RMS(9)   // 576
-        NCM_RMS(14)  // 896
-        NCM_RMS(16)
-        NCM_RMS(32)
-        NCM_RMS(40)  // 2560
-        NCM_RMS(64)
-        default: break;
+    const dim3 grid1((unsigned)((rows + 3) / 4));
+    if (n % 32 == 0 && n > kRmsRegMin && n <= kRmsRegMax) {
+        const bool few = rows <= kRmsFewRows;
+#define NCM_RMS(LOW, NR)                                                                        \
+    if (n <= 64 * NR) {                                                                        \
+        if (few)                                                                               \
+            hipLaunchKernelGGL((rms_norm_rows_reg_kernel<OUT_MODE, LOW, NR, true>), grid1,          \
+                               dim3(256), 0, stream, x, weight, y, rows, (int)n, epsilon);     \
+        else                                                                                   \
+            hipLaunchKernelGGL((rms_norm_rows_reg_kernel<OUT_MODE, LOW, NR, false>), grid1,         \
+                               dim3(256), 0, stream, x, weight, y, rows, (int)n, epsilon);     \
+        return hipGetLastError();                                                              \
     }
+        NCM_RMS(1, 2)
+        NCM_RMS(2, 4)
+        NCM_RMS(4, 6)
+        NCM_RMS(6, 8)
+        NCM_RMS(8, 10)
+        NCM_RMS(10, 12)
+        NCM_RMS(12, 14)
+        NCM_RMS(14, 16)
+        NCM_RMS(16, 20)
+        NCM_RMS(20, 24)
+        NCM_RMS(24, 28)
+        NCM_RMS(28, 32)
+        NCM_RMS(32, 40)
+        NCM_RMS(40, 48)
+        NCM_RMS(48, 56)
+        NCM_RMS(56, 64)
+        NCM_RMS(64, 80)
 #undef NCM_RMS
+    }
     // Wavefronts resident at once: 8 per SIMD on 256 CUs.
     constexpr int64_t kResidentWaves = 256 * 4 * 8;
     if (rows > kResidentWaves)
