@@ -88,6 +88,41 @@ def test_ncm_f32_body_matches_oracle(cuda, ncm, oracle, mask, hd, extras, window
     assert err.max() <= TOL * scale, err.max() / scale
 
 
+@pytest.mark.parametrize("mask,hd,levels,P", [
+    # 2048 keys of scores are kept at a time, 128 staged (64 past head_dim 128). The last
+    # level sees 2209 and 2080 keys: two walks. 130 prefix keys are three pad words, the prefix
+    # ends and the levels begin inside a stage and inside a workgroup's eight queries.
+    ("block_causal", 64, (9, 70, 300, 700, 1000), 130),
+    ("block_diagonal", 64, (40, 1950), 130),
+    ("block_diagonal", 32, (5, 1911, 60), 137),
+    # One walk, to the last score: 2048 keys.
+    ("block_causal", 64, (18, 900, 1000), 130),
+    ("block_causal", 160, (9, 70, 145), 70),
+    ("block_diagonal", 256, (3, 11, 90), 197),
+])
+def test_ncm_f32_level_mask_past_a_stage(cuda, ncm, oracle, mask, hd, levels, P):
+    """One layer whose level mask crosses the attention's stages and walks, with
+    a padded prefix. A key more or less among 2209 moves a context by some 4e-4
+    of a value, fp32 sums over so few layers by under 1e-6: bar 1e-5."""
+    from ncmorph_amd import ncm as N
+    import torch
+
+    print(f"ncm f32 level mask {mask} hd={hd} levels={levels} P={P}", flush=True)
+    rng = np.random.default_rng(hd + P)
+    hidden, vq, hq, hkv, inter, vocab = 64, 32, 2, 1, 64, 50
+    spec = _spec(N, levels, P, hidden, vq, hq, hkv, hd, inter, 1, mask, vocab)
+    w = random_ncm(rng, _ident, hidden, vq, inter, hq, hkv, hd, 1, list(levels), P, vocab)
+    ids = rng.integers(0, vocab, P)
+    pad = rng.random(P) < 0.3
+    pad[64:70] = True
+    tgt = rng.standard_normal((sum(levels), vq)).astype(np.float32)
+    got = _run(N, torch, cuda, spec, N.device_weights_f32(spec, w, cuda), ids, tgt, pad)
+    ref = oracle.ncm_forward(_cfg(spec), w, ids, pad, tgt, bf16=False, mask=mask)
+    err = np.abs(got - ref).max() / np.max(np.abs(ref))
+    print("max error relative to max|ref|:", err)
+    assert np.all(np.isfinite(got)) and err <= 1e-5, err
+
+
 def test_ncm_f32_hidden_states_match_oracle(cuda, ncm, oracle):
     """hidden_states in the reference's own arithmetic (forward_with_trace,
     src/ncm_model.zig:169-171, :243-249): [layers + 1, S, hidden], the
