@@ -293,14 +293,14 @@ hipError_t launch_slice(int tile, const SliceArgs& a, hipStream_t st) {
 // up to 1024: the 64 x 128 tiles take those (77 rows, 9728 x 576 / x 896: 9.6 -> 8.1 /
 // 11.6 -> 10.2 us; 150 rows, 6144 x 576 9.0 -> 8.1; 1100 rows, 1152 x 576 8.4 -> 7.5; but
 // 300 rows, 4096 x 1024 10.5 -> 11.4, 77 rows, 14336 x 4096 31.8 -> 33.9).
-constexpr int64_t kLargestTile = 9;  // cost of a round of the 5 x 4 tile
+constexpr int kLargestTile = kSliceTileCount - 1;
 
 bool linear_slice_fits(int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || N <= 0 || K <= 0 || K > (int64_t)1 << 21) return false;
     if (M <= 64) return true;
     int tile;
     const int64_t cost = best_tile(M, N, false, &tile);
-    if (cost == kLargestTile && (K <= 640 || (K <= 1024 && M <= 80))) return false;
+    if (tile == kLargestTile && (K <= 640 || (K <= 1024 && M <= 80))) return false;
     return cost <= 13;
 }
 

@@ -1,5 +1,6 @@
 """Few-row linears (csrc/linear_slice.hip: small tiles, K split over the
-wavefronts): every tile it chooses between, at M, N and K around its edges.
+wavefronts): every tile it chooses between, at M, N and K around its edges
+(test_linear_slice_choice.py holds these lists to that).
 
 Bars: every output within the D53 bound |y - y_f64| <= (K + 2) 2^-24 sum|x w|
 (+ |bias|) of float64 (packages/kernels/root.zig:96-142), and bit for bit: the
@@ -19,7 +20,30 @@ pytestmark = pytest.mark.gpu
 SHAPES = [(1, 8, 1), (1, 2048, 2048), (16, 72, 64), (17, 576, 576), (33, 1096, 130),
           (48, 520, 49153), (49, 64, 49153), (64, 4864, 897), (65, 896, 1152), (81, 2048, 3071),
           (130, 1536, 2048), (203, 1000, 2048), (300, 512, 2048), (512, 328, 2048),
-          (600, 136, 2047), (640, 24, 1000)]
+          (600, 136, 2047), (640, 24, 1000),
+          # 2 x 1, 1 x 2, 1 x 4, 2 x 2, 3 x 2, 4 x 2, 2 x 4, 3 x 4 and 5 x 4 blocks.
+          (20, 72, 2063), (3, 1000, 4113), (5, 264, 8209), (19, 72, 4113), (40, 136, 4113),
+          (50, 72, 4099), (65, 136, 4113), (70, 72, 5457), (130, 648, 5457)]
+FUSED = [(1, 64, 32), (17, 576, 1536), (33, 520, 24608), (64, 1096, 4864), (77, 256, 2048),
+         (203, 264, 1024),
+         # 2 x 2, 1 x 4, 2 x 4, 3 x 4 and 5 x 4 blocks, the last also at a model's size.
+         (20, 72, 2080), (5, 72, 4128), (19, 136, 4128), (35, 72, 4128), (130, 648, 2752), (77, 1096, 8192)]
+# K below, at and past one round of the wavefronts' 32-element tiles; N of one
+# and of several rounds; the last of the first line past the small tiles' range.
+F32 = [(1, 4, 1), (17, 576, 960), (33, 260, 1153), (77, 4864, 896), (200, 576, 577),
+       (300, 1000, 4864), (600, 36, 130), (130, 896, 20000),
+       (20, 36, 2113), (1, 36, 4161), (19, 36, 4161), (34, 36, 5505), (34, 36, 4161),
+       (50, 36, 4161), (67, 36, 4161), (67, 132, 5505), (100, 1000, 5505), (131, 260, 5505)]
+# hidden, intermediate, q heads, kv heads, head_dim, tokens of each of two
+# sequences, biases.
+DECODER_F32 = [(128, 256, 4, 2, 64, 37, True), (576, 1536, 9, 3, 64, 77, False),
+               (96, 68, 3, 1, 32, 20, True), (576, 1536, 9, 3, 64, 100, True),
+               (36, 4160, 63, 1, 64, 5, False), (36, 2112, 63, 1, 64, 10, True),
+               (36, 4160, 63, 1, 64, 10, True), (36, 4160, 63, 1, 64, 17, False),
+               (36, 2112, 63, 1, 64, 25, True), (36, 4160, 63, 1, 64, 25, False),
+               (36, 4160, 63, 1, 64, 34, True), (36, 2752, 84, 1, 64, 17, True),
+               (132, 4160, 84, 1, 64, 34, False), (260, 4160, 84, 1, 64, 65, True),
+               (1000, 4160, 84, 1, 64, 50, False)]
 
 
 def _dev(rng, shape, std, cuda):
@@ -56,8 +80,7 @@ def test_slice_outputs(ncm, cuda, m, k, n):
     assert torch.equal(kernels.linear_bf16(x2, w, bias=b)[m - 1], y[m - 1])
 
 
-@pytest.mark.parametrize("m,k,inter", [(1, 64, 32), (17, 576, 1536), (33, 520, 24608),
-                                       (64, 1096, 4864), (77, 256, 2048), (203, 264, 1024)])
+@pytest.mark.parametrize("m,k,inter", FUSED)
 @pytest.mark.parametrize("bias", [False, True])
 def test_slice_fused_epilogues(ncm, oracle, cuda, m, k, inter, bias):
     import torch
@@ -83,11 +106,7 @@ def test_slice_fused_epilogues(ncm, oracle, cuda, m, k, inter, bias):
     assert torch.equal(got.view(torch.int16), ref.view(torch.int16))
 
 
-# K below, at and past one round of the wavefronts' 32-element tiles; N of one
-# and of several rounds; the last one past the small tiles' range.
-@pytest.mark.parametrize("m,k,n", [(1, 4, 1), (17, 576, 960), (33, 260, 1153), (77, 4864, 896),
-                                   (200, 576, 577), (300, 1000, 4864), (600, 36, 130),
-                                   (130, 896, 20000)])
+@pytest.mark.parametrize("m,k,n", F32)
 def test_slice_f32(ncm, cuda, m, k, n):
     import torch
     from ncmorph_amd import kernels
@@ -102,9 +121,7 @@ def test_slice_f32(ncm, cuda, m, k, n):
     assert bool(((y.double() - ref).abs() <= bound).all())
 
 
-@pytest.mark.parametrize("hidden,inter,hq,hkv,hd,t,biases", [(128, 256, 4, 2, 64, 37, True),
-                                                             (576, 1536, 9, 3, 64, 77, False),
-                                                             (96, 68, 3, 1, 32, 20, True)])
+@pytest.mark.parametrize("hidden,inter,hq,hkv,hd,t,biases", DECODER_F32)
 def test_f32_decoder_fused_equals_traced(ncm, oracle, cuda, hidden, inter, hq, hkv, hd, t,
                                          biases):
     """Without a trace the f32 layers run one q|k|v product with the rotation,
