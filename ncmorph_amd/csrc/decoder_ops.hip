@@ -643,15 +643,15 @@ static hipError_t launch_rms_t(const float* x, const float* weight, void* y, int
     const dim3 grid1((unsigned)((rows + 3) / 4));
     if (n % 32 == 0 && n > kRmsRegMin && n <= kRmsRegMax) {
         const bool few = rows <= kRmsFewRows;
-#define NCM_RMS(LOW, NR)                                                                        \
-    if (n <= 64 * NR) {                                                                        \
-        if (few)                                                                               \
-            hipLaunchKernelGGL((rms_norm_rows_reg_kernel<OUT_MODE, LOW, NR, true>), grid1,          \
-                               dim3(256), 0, stream, x, weight, y, rows, (int)n, epsilon);     \
-        else                                                                                   \
-            hipLaunchKernelGGL((rms_norm_rows_reg_kernel<OUT_MODE, LOW, NR, false>), grid1,         \
-                               dim3(256), 0, stream, x, weight, y, rows, (int)n, epsilon);     \
-        return hipGetLastError();                                                              \
+#define NCM_RMS(LOW, NR)                                                                      \
+    if (n <= 64 * NR) {                                                                       \
+        if (few)                                                                              \
+            hipLaunchKernelGGL((rms_norm_rows_reg_kernel<OUT_MODE, LOW, NR, true>), grid1,    \
+                               dim3(256), 0, stream, x, weight, y, rows, (int)n, epsilon);    \
+        else                                                                                  \
+            hipLaunchKernelGGL((rms_norm_rows_reg_kernel<OUT_MODE, LOW, NR, false>), grid1,   \
+                               dim3(256), 0, stream, x, weight, y, rows, (int)n, epsilon);    \
+        return hipGetLastError();                                                             \
     }
         NCM_RMS(1, 2)
         NCM_RMS(2, 4)
