@@ -196,8 +196,8 @@ static hipError_t launch_linear_s(const uint16_t* x, const uint16_t* w, const ui
 // Tile configurations of the bf16 linear (index = NCM_LINEAR_TILE):
 //  0: 256x256x64, 8 waves (64x128 each, 2 per SIMD), direct-to-LDS loads,
 //     2 LDS stages; SCHED 8: loads and fragment reads interleaved between
-//     the MFMAs of the first two k-steps, barrier in the middle of the last
-//     k-step
+//     the MFMAs of the first two k-steps, barrier after 24 of the last k-step's
+//     32 MFMAs
 //  1: 128x128x64, 8 waves (32x64, 2 per SIMD), DMA, SCHED 8, 4 LDS stages,
 //     16x16x32 MFMAs
 //  2: 128x128x64, 4 waves, DMA, fences (SCHED 4), 2 stages: two workgroups

@@ -210,9 +210,9 @@ hipError_t launch_tied_head(const uint16_t* z, const uint16_t* cb, const float* 
     hipLaunchKernelGGL(tied_head_scale_kernel, dim3(levels), dim3(256), 0, st, a, scale);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    // The linear's tiles: 256 x 256 when the levels together fill three
-    // quarters of the CUs with them, else 128 x 128 with four LDS stages (at
-    // most about one tile per CU) or two (two workgroups per CU).
+    // 256 x 256 tiles when the levels together fill three quarters of the CUs
+    // with them, else 128 x 128 with four LDS stages (at most about one tile
+    // per CU) or two (two workgroups per CU).
     using H0 = GemmShape<256, 256, 64, 4, 2, 2, 8, true, 2, false, 1, 24, -1, true>;
     using H1 = GemmShape<128, 128, 64, 2, 2, 2, 8, true, 4>;
     using H2 = GemmShape<128, 128, 64, 2, 2, 2, 4, true>;

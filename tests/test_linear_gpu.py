@@ -176,15 +176,15 @@ def test_linear_zero_k_and_empty(ncm, cuda):
 
 
 @pytest.mark.parametrize("m,k,n", [
-    (200, 1096, 300),     # 128 x 128 tiles, four LDS stages
+    (200, 1096, 300),     # the few-row kernel, 16 x 16 tiles
     (2148, 1096, 5400),   # 256 x 256 tiles (198 of them)
-    (2148, 1096, 2800),   # 256 x 128 tiles (198 of them)
+    (2148, 1096, 2800),   # 128 x 256 tiles (187 of them)
 ])
 def test_linear_ragged_long_k_bias_modes_repeatable(ncm, cuda, m, k, n):
     """Ragged M and N, K not a multiple of the 64-wide K tile (partial last
     tile), bias, every output mode against the D53 bound and each other, and
-    identical bits over repeated launches; one shape per tile configuration
-    the automatic choice uses."""
+    identical bits over repeated launches; a shape of the few-row kernel and of
+    two tiles (the others: test_linear_tiles_gpu.py)."""
     import torch
     from ncmorph_amd import kernels
 
@@ -234,12 +234,12 @@ def test_linear_decoder_caller_shapes(ncm, oracle, cuda, m, n, k):
 @pytest.mark.parametrize("m,n,k", [
     (4096, 8192, 8),      # 256 x 256 tiles, 512 of them (two rounds), one K tile
     (4096, 8192, 200),    # the same with a partial last K tile
-    (2560, 3584, 64),     # 256 x 128 tiles (280): one K tile, fewer than the stages
-    (2560, 3584, 136),    # 256 x 128 with three K tiles, the last partial
+    (2560, 3584, 64),     # 256 x 256 tiles (140 of them): one K tile, fewer than the stages
+    (2560, 3584, 136),    # the same with three K tiles, the last partial
     (2560, 3584, 1024),
 ])
 def test_linear_multi_round_grids(ncm, cuda, m, n, k):
-    """Grids with more tiles than the CUs hold at once, short and partial K:
+    """Grids of two rounds and of half a round of the CUs, short and partial K:
     rows from every row tile against the D53 bound; the bf16 modes and the
     residual-fused form against the fp32 output."""
     import torch
