@@ -29,8 +29,16 @@ __attribute__((amdgpu_waves_per_eu(S::OCC, S::OCC))) void linear_kernel(const vo
     extern __shared__ __attribute__((aligned(16))) char lds[];
 
     // XCD-aware grouped tile order: a run of consecutive logical ids covers a
-    // group_m x tiles_n band, and each XCD receives one contiguous run.
-    const int logical = xcd_remap((int)blockIdx.x, (int)gridDim.x);
+    // group_m x tiles_n band, and each XCD receives one contiguous run. Large
+    // outputs with a residual and a short K, bound by those two streams, are the
+    // exception where the runs are uneven: on 256 x 256 tiles the band's tiles side
+    // by side on all XCDs stream better (remapped -> here: 2300 x 11008, K 576 / 1024 /
+    // 2048 122 -> 95, 139 -> 112, 178 -> 152 us; at K 4096 even). Not on 128 x 256 tiles
+    // (4749 x 4864 x 1024 72 -> 81) nor in small outputs (2328 x 896 x 896 11.7 -> 14.5).
+    const bool streams = HAS_RES && S::BM == 256 && S::BN == 256 &&
+                         M * N >= ((int64_t)1 << 24) && K <= 2048 && gridDim.x % 8 != 0;
+    const int logical =
+        streams ? (int)blockIdx.x : xcd_remap((int)blockIdx.x, (int)gridDim.x);
     const int per_group = group_m * tiles_n;
     const int g = logical / per_group;
     const int tiles_m = (int)((M + S::BM - 1) / S::BM);
