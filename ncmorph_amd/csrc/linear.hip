@@ -70,6 +70,19 @@ __attribute__((amdgpu_waves_per_eu(S::OCC, S::OCC))) void linear_kernel(const vo
         const int q = lane & 3;
         const int col4 = (lane & 31) & ~3;
         const int hrow = 4 * (lane >> 5) + q;
+        // The residual of a 32 x 32 block is loaded before the block before it is
+        // stored: a load issued after a store (y may be the residual) returns
+        // after it, and 32 such round trips a wavefront took 50 us.
+        f32x4_t res[2][4];
+        auto load_residual = [&](int t, f32x4_t (&r)[4]) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int64_t m = m0 + wm * S::WM + (t % S::MB) * 32 + 8 * i + hrow;
+                r[i] = *(const f32x4_t*)(residual + m * N + n0 + wn * S::WN +
+                                         (t / S::MB) * 32 + col4);
+            }
+        };
+        if constexpr (HAS_RES) load_residual(0, res[0]);
 #pragma unroll
         for (int nb = 0; nb < S::NB; ++nb) {
             float bv = 0.0f;
@@ -77,6 +90,9 @@ __attribute__((amdgpu_waves_per_eu(S::OCC, S::OCC))) void linear_kernel(const vo
             const int64_t ncol = n0 + wn * S::WN + nb * 32 + col4;
 #pragma unroll
             for (int mb = 0; mb < S::MB; ++mb) {
+                const int t = nb * S::MB + mb;
+                if constexpr (HAS_RES)
+                    if (t + 1 < S::NB * S::MB) load_residual(t + 1, res[(t + 1) & 1]);
 #pragma unroll
                 for (int blk = 0; blk < 4; ++blk) {
                     float v[4];
@@ -87,8 +103,7 @@ __attribute__((amdgpu_waves_per_eu(S::OCC, S::OCC))) void linear_kernel(const vo
                     }
                     quad_transpose4(v, q);
                     const int64_t m = m0 + wm * S::WM + mb * 32 + 8 * blk + hrow;
-                    f32x4_t rv;
-                    if (HAS_RES) rv = *(const f32x4_t*)(residual + m * N + ncol);
+                    const f32x4_t rv = res[t & 1][blk];
                     if (OUT_MODE == NCM_OUT_F32) {
                         f32x4_t o;
                         o[0] = v[0]; o[1] = v[1]; o[2] = v[2]; o[3] = v[3];
@@ -132,26 +147,45 @@ __attribute__((amdgpu_waves_per_eu(S::OCC, S::OCC))) void linear_kernel(const vo
         }
         return;
     }
+    // A partial tile, element by element; the residual ahead as above.
+    float res[2][16];
+    auto row_of = [&](int mb, int i) {
+        return m0 + wm * S::WM + mb * 32 + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
+    };
+    auto load_residual = [&](int t, float (&r)[16]) {
+        const int64_t n = n0 + wn * S::WN + (t / S::MB) * 32 + (lane & 31);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const int64_t m = row_of(t % S::MB, i);
+            r[i] = n < N && m < M ? residual[m * N + n] : 0.0f;
+        }
+    };
+    if constexpr (HAS_RES) load_residual(0, res[0]);
 #pragma unroll
     for (int nb = 0; nb < S::NB; ++nb) {
         const int64_t n = n0 + wn * S::WN + nb * 32 + (lane & 31);
-        if (n >= N) continue;
+        if (!HAS_RES && n >= N) continue;  // with a residual the next block's loads come first
         float bv = 0.0f;
-        if (HAS_BIAS) bv = __uint_as_float((uint32_t)bias[n] << 16);
+        if (HAS_BIAS && n < N) bv = __uint_as_float((uint32_t)bias[n] << 16);
 #pragma unroll
         for (int mb = 0; mb < S::MB; ++mb) {
+            const int t = nb * S::MB + mb;
+            if constexpr (HAS_RES) {
+                if (t + 1 < S::NB * S::MB) load_residual(t + 1, res[(t + 1) & 1]);
+                if (n >= N) continue;
+            }
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
-                const int64_t m =
-                    m0 + wm * S::WM + mb * 32 + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
+                const int64_t m = row_of(mb, i);
                 if (m >= M) continue;
                 float v = acc.v[mb][nb][i];
                 if (HAS_BIAS) v = v + bv;
+                const float rv = res[t & 1][i];
                 if (OUT_MODE == NCM_OUT_F32) {
-                    ((float*)y)[m * N + n] = HAS_RES ? residual[m * N + n] + v : v;
+                    ((float*)y)[m * N + n] = HAS_RES ? rv + v : v;
                 } else {
                     uint32_t bits = bf16_bits_rne(flush_subnormal(v));
-                    if (HAS_RES) bits = bf16_bits_rne(residual[m * N + n] + __uint_as_float(bits << 16));
+                    if (HAS_RES) bits = bf16_bits_rne(rv + __uint_as_float(bits << 16));
                     if (OUT_MODE == NCM_OUT_BF16_F32)
                         ((float*)y)[m * N + n] = __uint_as_float(bits << 16);
                     else
