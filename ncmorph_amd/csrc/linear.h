@@ -13,6 +13,15 @@ int linear_tile_config(int64_t M, int64_t N, int forced);
 // (128x128), and its cost: 100 is a full round of 256x256 tiles.
 constexpr int kTile128x256 = 16, kTile64x128 = 17;
 int64_t linear_tile_cost(int64_t M, int64_t N, int* tile);
+// Row tiles per band of the tile order (linear_kernel): four, and five where a
+// band of one would be left over after one or two: it reads the whole weight
+// again, on one or two XCDs (64x128 tiles, 300 rows: 6144 x 4096 28.9 -> 20 us,
+// 12288 x 8192 106 -> 74; 128x256, 600 rows: 28672 x 1024 57 -> 50; 256x256, 2200 rows:
+// 4096 x 4096 87 -> 84; from 17 row tiles on longer bands cost up to 4%).
+inline int linear_band(int tiles_m) {
+    if (tiles_m == 5 || tiles_m == 9) return 5;
+    return tiles_m < 4 ? tiles_m : 4;
+}
 
 hipError_t launch_linear(const uint16_t* x, const uint16_t* w, const uint16_t* bias, void* y,
                          int64_t M, int64_t K, int64_t N, int out_mode, int config,

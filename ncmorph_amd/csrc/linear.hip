@@ -211,7 +211,7 @@ static hipError_t launch_linear_t(const void* x, const void* w, const uint16_t* 
     }
     const int tiles_m = (int)((M + S::BM - 1) / S::BM);
     const int tiles_n = (int)((N + S::BN - 1) / S::BN);
-    const int group_m = tiles_m < 4 ? tiles_m : 4;
+    const int group_m = linear_band(tiles_m);
     hipLaunchKernelGGL(kern, dim3(tiles_m * tiles_n), dim3(S::NT), S::LDS_BYTES, stream, x, w,
                        bias, y, M, K, N, tiles_n, group_m, residual);
     return hipGetLastError();
