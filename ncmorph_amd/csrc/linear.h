@@ -9,8 +9,8 @@ namespace ncm {
 // Tile configuration chosen for an M x N output (see the table in
 // linear.hip); a valid `forced` index overrides the choice.
 int linear_tile_config(int64_t M, int64_t N, int forced);
-// The automatic choice's tiles besides configurations 0 (256x256) and 1
-// (128x128), and its cost: 100 is a full round of 256x256 tiles.
+// The automatic choice's tiles besides configurations 0 (256x256), 1 (128x128)
+// and 5 (256x128), and its cost: 1000 is a full round of 256x256 tiles.
 constexpr int kTile128x256 = 16, kTile64x128 = 17;
 int64_t linear_tile_cost(int64_t M, int64_t N, int* tile);
 // Row tiles per band of the tile order (linear_kernel): four, and five where a

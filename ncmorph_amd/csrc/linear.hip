@@ -30,13 +30,14 @@ __attribute__((amdgpu_waves_per_eu(S::OCC, S::OCC))) void linear_kernel(const vo
 
     // XCD-aware grouped tile order: a run of consecutive logical ids covers a
     // group_m x tiles_n band, and each XCD receives one contiguous run. Large
-    // outputs with a residual and a short K, bound by those two streams, are the
-    // exception where the runs are uneven: on 256 x 256 tiles the band's tiles side
-    // by side on all XCDs stream better (remapped -> here: 2300 x 11008, K 576 / 1024 /
-    // 2048 122 -> 95, 139 -> 112, 178 -> 152 us; at K 4096 even). Not on 128 x 256 tiles
-    // (4749 x 4864 x 1024 72 -> 81) nor in small outputs (2328 x 896 x 896 11.7 -> 14.5).
-    const bool streams = HAS_RES && S::BM == 256 && S::BN == 256 &&
-                         M * N >= ((int64_t)1 << 24) && K <= 2048 && gridDim.x % 8 != 0;
+    // outputs of a short K, bound by their stores (and residual), are the exception
+    // where the runs are uneven: on 256 x 256 tiles the band's tiles side by side on
+    // all XCDs stream better (remapped -> here: 2300 x 11008 with a residual, K 576 /
+    // 1024 / 2048 122 -> 95, 139 -> 112, 178 -> 152 us, at K 4096 even; 2700 x 9728 x 896 71 ->
+    // 63, 1400 x 151936 x 896 502 -> 489, at K 2048 even). Not on 128 x 256 tiles (4749 x
+    // 4864 x 1024 72 -> 81) nor in small outputs (2328 x 896 x 896 11.7 -> 14.5).
+    const bool streams = S::BM == 256 && S::BN == 256 && M * N >= ((int64_t)1 << 24) &&
+                         K <= (HAS_RES ? 2048 : 1024) && gridDim.x % 8 != 0;
     const int logical =
         streams ? (int)blockIdx.x : xcd_remap((int)blockIdx.x, (int)gridDim.x);
     const int per_group = group_m * tiles_n;
@@ -289,32 +290,40 @@ constexpr int kLinConfigs = 16;
 using LinF32 = GemmShape<128, 128, 32, 2, 2, 2, 5, true, 2, true>;
 using LinF32Small = GemmShape<64, 64, 32, 2, 2, 4, 8, true, 2, true>;
 
-// The tile of an M x N product: the least number of rounds of the 256 CUs
-// times the time of a round, relative to a round of 256x256 tiles. Measured (K 576
-// .. 8192, M 70 .. 6000, N 2048 .. 151936), a round of 256x256 at K 2048 takes 45 us,
-// of 128x256 24 and in products of many rounds 27, of 128x128 14-18, of 64x128 11.
-// All four sum in the same order, so the choice does not change a bit.
+// The tile of an M x N product: the least time, in thousandths of a round of
+// 256x256 tiles on the 256 CUs (45 us at K 2048). A last round of few tiles has the
+// memory to itself: it takes 0.65 of a full one and more as it fills, or 0.9 and more
+// where it is the only one. Fitted with weights that come from HBM, as a model's do
+// (391 products of M 70 .. 4096, the projections of five checkpoints): 0.7% from
+// the best of the five tiles in the mean. All sum in the same order, so the choice does
+// not change a bit.
 //
-// Where the choice falls, 256x256 (three quarters of a round or more), 256x128 or
-// 128x128 with two stages -> here, us: 77 rows of 128256 x 2048 164 -> 136 and of
-// 151936 x 1024 120 -> 81 (256-row tiles multiply 179 rows of padding), 300 rows
-// 253 -> 220 and 175 -> 148 (384 rows instead of 512), 700 of 28672 x 4096 185 ->
-// 153, 1500 of 16384 x 2048 113 -> 95 (3 rounds of halves for 2), 300 of 3072 x 2048
-// 15.4 -> 12.1, 1000 of 2048 x 8192 48 -> 40.
+// 256x128 against 128x256: the weight passes half as many row tiles, worth up to
+// 17% while it streams from HBM (384 x 14336 x 4096 57 us against 67, 850 x 6144 x 4096
+// 48 against 56, 1500 x 4096 x 14336 175 against 190) and -6 .. +2% from the
+// memory-side cache; 128x256 where it pads fewer rows. The two and 64x128 against
+// 256x256 (three quarters of a round or more) and 128x128 with two stages alone, us: 77
+// rows of 128256 x 2048 164 -> 136 and of 151936 x 1024 120 -> 81 (256-row tiles multiply
+// 179 rows of padding), 300 rows 253 -> 220 and 175 -> 148 (384 rows instead of 512), 1500
+// of 16384 x 2048 113 -> 95 (3 rounds of halves for 2), 300 of 3072 x 2048 15.4 -> 12.1.
 struct TileCost {
     int bm, bn, cost, tile;
 };
-constexpr TileCost kTiles[] = {{256, 256, 100, 0},
-                               {128, 256, 59, kTile128x256},
-                               {128, 128, 35, 1},
-                               {64, 128, 25, kTile64x128}};
+constexpr TileCost kTiles[] = {{256, 256, 1000, 0},
+                               {256, 128, 540, 5},
+                               {128, 256, 580, kTile128x256},
+                               {128, 128, 350, 1},
+                               {64, 128, 270, kTile64x128}};
 constexpr int64_t kTileCus = 256;
 
 int64_t linear_tile_cost(int64_t M, int64_t N, int* tile) {
     int64_t best = INT64_MAX;
     for (const TileCost& t : kTiles) {
         const int64_t n = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
-        const int64_t c = ((n + kTileCus - 1) / kTileCus) * t.cost;
+        const int64_t full = n / kTileCus, rest = n % kTileCus;
+        int64_t c = full * 1000;
+        if (rest > 0) c += full > 0 ? 650 + 350 * rest / kTileCus : 900 + 100 * rest / kTileCus;
+        c = c * t.cost / 1000;
         if (c < best) {
             best = c;
             *tile = t.tile;
@@ -412,6 +421,7 @@ hipError_t launch_linear_residual(const uint16_t* x, const uint16_t* w, const ui
     switch (linear_tile_config(M, N, -1)) {
         case 0: return launch_linear_res_s<Lin0>(x, w, bias, residual, y, M, K, N, out_mode, stream);
         case 1: return launch_linear_res_s<Lin1>(x, w, bias, residual, y, M, K, N, out_mode, stream);
+        case 5: return launch_linear_res_s<Lin5>(x, w, bias, residual, y, M, K, N, out_mode, stream);
         case kTile128x256:
             return launch_linear_res_s<Lin128x256>(x, w, bias, residual, y, M, K, N, out_mode,
                                                    stream);

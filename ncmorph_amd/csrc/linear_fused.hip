@@ -211,6 +211,7 @@ static hipError_t launch_pair(const uint16_t* x, const uint16_t* w, const uint16
                               hipStream_t st) {
     using L0 = GemmShape<256, 256, 64, 4, 2, 2, 8, true, 2, false, 1, 24, -1, true>;
     using L1 = GemmShape<128, 128, 64, 4, 2, 2, 8, true, 4, false, 1, -1, -1, true>;
+    using L5 = GemmShape<256, 128, 64, 4, 2, 2, 8, true, 3, false, 1, -1, -1, true>;
     using L128x256 = GemmShape<128, 256, 64, 2, 4, 2, 8, true, 3, false, 1, -1, -1, true>;
     using L64x128 = GemmShape<64, 128, 64, 2, 2, 2, 8, true, 4, false, 1, -1, -1, true>;
     const bool hb = bias != nullptr;
@@ -221,6 +222,9 @@ static hipError_t launch_pair(const uint16_t* x, const uint16_t* w, const uint16
         case 1:
             return hb ? launch_pair_t<L1, EPI, true>(x, w, bias, y, M, K, N, pa, st)
                       : launch_pair_t<L1, EPI, false>(x, w, bias, y, M, K, N, pa, st);
+        case 5:
+            return hb ? launch_pair_t<L5, EPI, true>(x, w, bias, y, M, K, N, pa, st)
+                      : launch_pair_t<L5, EPI, false>(x, w, bias, y, M, K, N, pa, st);
         case kTile128x256:
             return hb ? launch_pair_t<L128x256, EPI, true>(x, w, bias, y, M, K, N, pa, st)
                       : launch_pair_t<L128x256, EPI, false>(x, w, bias, y, M, K, N, pa, st);

@@ -275,7 +275,7 @@ int64_t linear_tail_rows(int64_t M, int64_t N, int64_t K) {
     int tile_all, tile_main;
     const int64_t all = linear_tile_cost(M, N, &tile_all);
     const int64_t main = linear_tile_cost(M - r, N, &tile_main);
-    return tile_main == 0 && main + 10 + N / 500 < all ? r : 0;
+    return tile_main == 0 && main + 100 + N / 50 < all ? r : 0;
 }
 
 hipError_t launch_linear_tail(const uint16_t* x, const uint16_t* w, const uint16_t* bias,

@@ -178,7 +178,7 @@ def test_linear_zero_k_and_empty(ncm, cuda):
 @pytest.mark.parametrize("m,k,n", [
     (200, 1096, 300),     # the few-row kernel, 16 x 16 tiles
     (2148, 1096, 5400),   # 256 x 256 tiles (198 of them)
-    (2148, 1096, 2800),   # 128 x 256 tiles (187 of them)
+    (2148, 1096, 2800),   # 256 x 128 tiles (198 of them)
 ])
 def test_linear_ragged_long_k_bias_modes_repeatable(ncm, cuda, m, k, n):
     """Ragged M and N, K not a multiple of the 64-wide K tile (partial last

@@ -22,12 +22,13 @@ def _dev(rng, shape, std, cuda):
 
 
 # 64x128 (one round, two row tiles and six), 128x256 (one row tile, three, two
-# rounds), 128x128 (one round and three), 256x256 (the last with the residual's
-# own tile order: 2^24 elements or more, a grid that is no multiple of 8). Five row
-# tiles (one band) of 64x128 and 128x256, nine of 256x256.
+# rounds), 128x128, 256x256, 256x128 (three row tiles, nine in three rounds). Five row
+# tiles (one band) of 64x128 and 128x256, nine of 256x256; the last with the
+# residual's own tile order (2^24 elements or more, a grid that is no multiple of 8).
 @pytest.mark.parametrize("m,k,n", [(128, 136, 16383), (350, 72, 5000), (77, 520, 9999), (128, 64, 49153),
                                    (300, 328, 40001), (1100, 8, 14000), (1500, 72, 2049), (600, 72, 15900),
-                                   (600, 520, 9000), (2047, 200, 8190), (2300, 72, 7400), (300, 72, 6143)])
+                                   (600, 520, 9000), (2047, 200, 8190), (2300, 72, 7400), (300, 72, 6143),
+                                   (600, 72, 12800), (2300, 72, 12000)])
 def test_tile_outputs(ncm, cuda, m, k, n):
     import torch
     from ncmorph_amd import kernels
@@ -59,7 +60,7 @@ def test_tile_outputs(ncm, cuda, m, k, n):
 
 @pytest.mark.parametrize("m,k,inter", [(128, 136, 8192 - 32), (350, 72, 2560), (128, 64, 24608),
                                        (300, 200, 20000), (1100, 72, 7008), (1500, 64, 1056),
-                                       (300, 72, 3072)])
+                                       (300, 72, 3072), (600, 72, 4512)])
 @pytest.mark.parametrize("bias", [False, True])
 def test_tile_fused_epilogues(ncm, oracle, cuda, m, k, inter, bias):
     import torch
