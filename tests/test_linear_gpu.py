@@ -234,12 +234,12 @@ def test_linear_decoder_caller_shapes(ncm, oracle, cuda, m, n, k):
 @pytest.mark.parametrize("m,n,k", [
     (4096, 8192, 8),      # 256 x 256 tiles, 512 of them (two rounds), one K tile
     (4096, 8192, 200),    # the same with a partial last K tile
-    (2560, 3584, 64),     # 256 x 256 tiles (140 of them): one K tile, fewer than the stages
-    (2560, 3584, 136),    # the same with three K tiles, the last partial
+    (2560, 3584, 64),     # 256 x 128 tiles (280): one K tile, fewer than the stages
+    (2560, 3584, 136),    # 256 x 128 with three K tiles, the last partial
     (2560, 3584, 1024),
 ])
 def test_linear_multi_round_grids(ncm, cuda, m, n, k):
-    """Grids of two rounds and of half a round of the CUs, short and partial K:
+    """Grids with more tiles than the CUs hold at once, short and partial K:
     rows from every row tile against the D53 bound; the bf16 modes and the
     residual-fused form against the fp32 output."""
     import torch
